@@ -64,7 +64,7 @@ def tune(policies=("crout_ref", "abs"), ns=range(1, 65), target_mib: int = 256, 
         for n in ns:
             cnt = count or int(min(262144, max(4096, (target_mib << 20) // (16 * n * n))))
             A = wl.gaussian(cnt, n, seed + n, device=dev)
-            res = lc.alloc_result(count, n, dev)
+            res = lc.alloc_result(cnt, n, dev)
             ref = None
             times = []
             for shape in range(lc.shape_count(n)):

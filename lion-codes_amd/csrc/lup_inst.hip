@@ -7,6 +7,7 @@
 
 #include "lup_dispatch.hpp"
 #include "lup_kernel.hpp"
+#include "lup_panel.hpp"
 
 #if !defined(LUFQHE_VARIANT) || !defined(LUFQHE_SHARD) || !defined(LUFQHE_SHARDS)
 #error "compile with -DLUFQHE_VARIANT=v -DLUFQHE_SHARD=s -DLUFQHE_SHARDS=k"
@@ -22,23 +23,37 @@ constexpr int kArith = variant_arith(LUFQHE_VARIANT);
 constexpr int kWavesPerBlock = 1;
 
 template <int N, int SH>
+constexpr ShapeLC shape_of() {
+  return kArith == ARITH_FUSED ? candidate_shape(N, SH) : reference_shape(N);
+}
+
+template <int N, int SH>
+constexpr auto kernel_of() {
+  constexpr ShapeLC sh = shape_of<N, SH>();
+  if constexpr (sh.panel)
+    return &lup_panel_kernel<N, 64 / sh.lanes, kPolicy, sh.waves>;
+  else
+    return &lup_det_kernel<N, sh.lanes, sh.lane_cols, kPolicy, kArith, kWavesPerBlock, sh.waves>;
+}
+
+template <int N, int SH>
 hipError_t launch(const BatchArgs& args, int64_t blocks, hipStream_t stream) {
-  constexpr ShapeLC sh = candidate_shape(N, SH);
-  hipLaunchKernelGGL((lup_det_kernel<N, sh.lanes, sh.lane_cols, kPolicy, kArith, kWavesPerBlock, sh.waves>),
-                     dim3((unsigned)blocks), dim3(64 * kWavesPerBlock), 0, stream, args);
+  hipLaunchKernelGGL((kernel_of<N, SH>()), dim3((unsigned)blocks), dim3(64 * kWavesPerBlock), 0,
+                     stream, args);
   return hipGetLastError();
 }
 
 template <int N, int SH>
 void register_shape() {
-  constexpr ShapeLC sh = candidate_shape(N, SH);
-  // reference arithmetic is a parity mode: only its default shape is built
+  constexpr ShapeLC sh = shape_of<N, SH>();
+  // reference arithmetic is a parity mode: only one shape is built
   if constexpr (sh.lanes > 0 && (kArith == ARITH_FUSED || SH == 0)) {
+    static_assert(!sh.panel || (sh.lanes == 64 / panel_groups(N) && sh.lane_cols == 4),
+                  "the panel kernel's geometry");
     KernelEntry& e = g_kernels[LUFQHE_VARIANT][N][SH];
     e.launch = &launch<N, SH>;
     e.shape = KernelShape{sh.lanes, sh.lane_cols, kWavesPerBlock, sh.waves};
-    e.kernel = reinterpret_cast<const void*>(
-        &lup_det_kernel<N, sh.lanes, sh.lane_cols, kPolicy, kArith, kWavesPerBlock, sh.waves>);
+    e.kernel = reinterpret_cast<const void*>(kernel_of<N, SH>());
   }
 }
 

@@ -902,9 +902,9 @@ __device__ __forceinline__ void write_result(const DetOut& out, int64_t m,
     ph = 0.0;
     mx = my = 0.0;
     e = 0;
-  } else {
-    la = 0.5 * log(fma(mx, mx, my * my)) + (double)e * kLn2;
-    ph = atan2(my, mx);
+  } else {  // a caller of (mant, exp) alone does not pay for the logarithm
+    la = out.logabs ? 0.5 * log(fma(mx, mx, my * my)) + (double)e * kLn2 : 0.0;
+    ph = out.phase ? atan2(my, mx) : 0.0;
   }
   out.mant[m] = make_double2(mx, my);
   if (out.expo) out.expo[m] = e;
@@ -1048,51 +1048,64 @@ __global__ void __launch_bounds__(64 * WPB, OCC) lup_det_kernel(BatchArgs args) 
 }
 
 // Candidate launch shapes per n, as (lanes per matrix L, lane-columns CG,
-// waves per SIMD the register allocation must allow).  Every candidate is
-// compiled; the autotuner picks one per n on the device and candidate 0 is
-// the default before tuning.  The lists come from shape sweeps on MI355X:
-// small n wants many matrices per wave (even two rows per lane), mid n a
-// split of each row over lane-columns, n > 40 one matrix per wave.  Up to
-// n = 40 the natural allocation sits just under or just over 256 VGPRs, so
-// those candidates are capped at 256 (two waves per SIMD).  From n = 41 the
-// tile alone needs 100-256 VGPRs and the natural allocation leaves one wave
-// per SIMD, which cannot hide the step's dependent latencies; the waves = 2
-// candidates cap the allocation at 256 registers (spilling the coldest
-// values to scratch), which measured up to 1.6x faster at n = 48.
+// waves per SIMD the register allocation must allow, panel kernel or not).
+// Every candidate is compiled; the autotuner picks one per n on the device
+// and candidate 0 is the default before tuning.  The lists come from shape
+// sweeps on MI355X (about 512 MiB of matrices, ns per determinant): small n
+// wants many matrices per wave (even two rows per lane), n = 17..24 a split of
+// each row over lane-columns.  The panel kernel (lup_panel.hpp) takes a fixed
+// lane per row of its panel, so it loses where rows are few (n = 17: 2.57
+// against 1.97, n = 20: 2.92 against 2.45), wins at odd n in between (n = 23:
+// 3.67 against 4.77) and from n = 25 on (n = 32: 6.8 against 7.8, n = 48: 19.8
+// against 26.0, n = 64: 50 against 81), so from n = 33 it is the only one.
+// Two waves per SIMD hide its serial steps; above n = 48 that costs spills of
+// the first panels' slots, which still pays at n = 56 (35.1 against 38.6) and
+// no longer at n = 64 (52.8 against 49.4).
 struct ShapeLC {
   int lanes;
   int lane_cols;
   int waves;
+  bool panel;
 };
 constexpr int kMaxShapes = 4;
 constexpr ShapeLC candidate_shape(int n, int idx) {
-  constexpr ShapeLC none{0, 0, 0};
+  constexpr ShapeLC none{0, 0, 0, false};
   if (n <= 8) {
-    constexpr ShapeLC c[] = {{4, 1, 1}, {8, 1, 1}, none, none};
+    constexpr ShapeLC c[] = {{4, 1, 1, false}, {8, 1, 1, false}, none, none};
     return c[idx];
   }
   if (n <= 16) {
-    constexpr ShapeLC c[] = {{16, 1, 1}, {8, 1, 1}, none, none};
+    constexpr ShapeLC c[] = {{16, 1, 1, false}, {8, 1, 1, false}, none, none};
     return c[idx];
   }
   if (n <= 24) {
-    constexpr ShapeLC c[] = {{32, 4, 2}, {16, 2, 2}, {32, 2, 2}, none};
+    constexpr ShapeLC c[] = {{32, 4, 2, false}, {16, 2, 2, false}, {32, 2, 2, false}, {32, 4, 3, true}};
     return c[idx];
   }
   if (n <= 32) {
-    constexpr ShapeLC c[] = {{32, 2, 2}, {32, 4, 2}, {32, 1, 2}, none};
+    constexpr ShapeLC c[] = {{32, 4, 2, true}, {32, 2, 2, false}, {32, 1, 2, false}, none};
     return c[idx];
   }
   if (n <= 40) {
-    constexpr ShapeLC c[] = {{64, 4, 2}, {64, 1, 2}, {64, 2, 2}, none};
+    constexpr ShapeLC c[] = {{64, 4, 2, true}, {64, 4, 3, true}, none, none};
     return c[idx];
   }
   if (n <= 48) {
-    constexpr ShapeLC c[] = {{64, 4, 2}, {64, 2, 2}, {64, 4, 1}, {32, 4, 1}};
+    constexpr ShapeLC c[] = {{64, 4, 2, true}, none, none, none};
     return c[idx];
   }
-  constexpr ShapeLC c[] = {{64, 2, 1}, {64, 4, 1}, {64, 4, 2}, {64, 2, 2}};
+  constexpr ShapeLC c[] = {{64, 4, 2, true}, {64, 4, 1, true}, none, none};
   return c[idx];
+}
+
+// The one shape of the reference-arithmetic variant.
+constexpr ShapeLC reference_shape(int n) {
+  if (n <= 8) return {4, 1, 1, false};
+  if (n <= 16) return {16, 1, 1, false};
+  if (n <= 24) return {32, 4, 2, false};
+  if (n <= 32) return {32, 2, 2, false};
+  if (n <= 48) return {64, 4, 2, false};
+  return {64, 2, 1, false};
 }
 
 }  // namespace lufqhe

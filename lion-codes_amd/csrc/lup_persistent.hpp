@@ -7,8 +7,8 @@
 // class from a device work counter (one vector atomic per task), finds the
 // task's bucket -- buckets are ordered largest n first, so the large
 // matrices start first and the small ones fill the tail -- and factors the
-// task's matrices with that n's fully unrolled code (det_task, the same code
-// the per-size kernels run, so the results are bit-identical).  A wave leaves
+// task's matrices with that n's fully unrolled code (det_task or panel_task,
+// the code the per-size kernels run, so the results are bit-identical).  A wave leaves
 // the loop when the counter has passed the class's last task.
 //
 // A class kernel carries the register allocation of its largest case, so
@@ -20,6 +20,7 @@
 #pragma once
 
 #include "lup_kernel.hpp"
+#include "lup_panel.hpp"
 
 namespace lufqhe {
 
@@ -40,21 +41,21 @@ constexpr int persist_class(int n) {
 struct PersistShape {
   int lanes;
   int lane_cols;
+  bool panel;
 };
 constexpr PersistShape persist_shape(int n) {
-  if (n <= 8) return {4, 1};
-  if (n <= 16) return {8, 1};
-  if (n <= 24) return {16, 2};
-  if (n <= 32) return {32, 2};
-  if (n <= 48) return {64, 4};
-  return {64, 2};
+  if (n <= 8) return {4, 1, false};
+  if (n <= 16) return {8, 1, false};
+  if (n <= 24) return {16, 2, false};
+  if (n <= 32) return {32, 4, true};
+  return {64, 4, true};
 }
 constexpr int persist_group(int n) { return 64 / persist_shape(n).lanes; }  // matrices per task
 
-// LDS one task of size n uses (G groups of group_lds).
+// LDS one task of size n uses.
 constexpr int persist_lds(int n) {
   const PersistShape s = persist_shape(n);
-  return (64 / s.lanes) * group_lds(n, s.lanes, s.lane_cols);
+  return s.panel ? panel_lds(n) : (64 / s.lanes) * group_lds(n, s.lanes, s.lane_cols);
 }
 constexpr int persist_lds_max(int lo, int hi) {
   int m = 0;
@@ -89,7 +90,10 @@ __device__ __forceinline__ void persist_dispatch(int n, const BatchArgs& args, i
                                                  double2* __restrict__ bc, int lane) {
   if (n == N) {
     constexpr PersistShape s = persist_shape(N);
-    det_task<N, s.lanes, s.lane_cols, POLICY, ARITH_FUSED>(args, task, bc, lane);
+    if constexpr (s.panel)
+      panel_task<N, 64 / s.lanes, POLICY>(args, task, bc, lane);
+    else
+      det_task<N, s.lanes, s.lane_cols, POLICY, ARITH_FUSED>(args, task, bc, lane);
     return;
   }
   if constexpr (N < HI) persist_dispatch<N + 1, HI, POLICY>(n, args, task, bc, lane);

@@ -1,0 +1,84 @@
+"""The panel kernels (lion-codes_amd/csrc/lup_panel.hpp) where they can go
+wrong: sizes at the edges of their panels, row slots and matrices per wave,
+columns whose criteria tie in the upper word or exactly, criteria outside the
+corrected quotient's range, zero pivots and non-finite entries in the middle
+of a panel.  Every compiled launch shape of each size equals the oracle's
+mirror bit for bit (mantissa, exponent, pivots, status); a NaN mantissa need
+only be NaN on both sides, and a zero determinant has no sign."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SIZES = (17, 20, 21, 24, 25, 28, 29, 31, 32, 33, 36, 37, 48, 49, 52, 53, 61, 63, 64)
+
+
+def same(g, o):
+    o = np.where(o == 0, 0.0 + 0.0j, o)  # a zero determinant is written as +0 + 0i
+    g = np.ascontiguousarray(g).view(np.float64)
+    o = np.ascontiguousarray(o).view(np.float64)
+    return bool(((g.view(np.uint64) == o.view(np.uint64)) | (np.isnan(g) & np.isnan(o))).all())
+
+
+def check(lc, orc, dev, A):
+    n = A.shape[1]
+    d = torch.from_numpy(np.ascontiguousarray(A)).to(dev)
+    for policy in ("crout_ref", "abs"):
+        o = orc.mirror(A, policy, "fused")
+        keep = lc.get_shape(policy, "fused", n)
+        try:
+            for shape in range(lc.shape_count(n)):
+                assert lc.set_shape(policy, "fused", n, shape)
+                r = lc.det_batched(d, policy=policy, pivots=True)
+                torch.cuda.synchronize()
+                what = (n, policy, shape)
+                assert np.array_equal(r.info.cpu().numpy(), o["info"]), what
+                assert same(r.mant.cpu().numpy(), o["mant"]), what
+                assert np.array_equal(r.exp.cpu().numpy(), o["exp"]), what
+                ok = o["info"] >= 0
+                assert np.array_equal(r.piv.cpu().numpy()[ok].astype(np.int32), o["piv"][ok]), what
+        finally:
+            lc.set_shape(policy, "fused", n, keep)
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_batches_that_do_not_fill_a_wave(lc, orc, wl, dev, n):
+    for count in (1, 2, 3, 67):
+        check(lc, orc, dev, wl.gaussian_np(count, n, seed=10 * n + count))
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_ties_and_zero_pivots(lc, orc, wl, dev, n):
+    rng = np.random.default_rng(n)
+    ints = rng.integers(-2, 3, (9, n, n)) + 1j * rng.integers(-2, 3, (9, n, n))
+    ints[:, :, 0].real[:, ::2] = 2  # equal criteria in the first column
+    perm = np.zeros((4, n, n), np.complex128)
+    for m in range(4):
+        perm[m, np.arange(n), rng.permutation(n)] = rng.choice([1, -1, 2, 1 + 1j], n)
+    rank = ints[:3].copy()
+    rank[0, :, n // 2] = rank[0, :, n // 2 - 1]  # zero pivots inside and at the ends of panels
+    rank[1, n - 1] = rank[1, 0]
+    rank[2, :, 5] = 0
+    # upper words of the criteria equal, lower words deciding
+    close = np.tile(wl.gaussian_np(3, 1, seed=n), (1, n, n)) * (1 + 1e-9 * rng.standard_normal((3, n, n)))
+    check(lc, orc, dev, np.concatenate([ints, perm, rank, close]).astype(np.complex128))
+
+
+@pytest.mark.parametrize("n", [17, 28, 32, 33, 48, 52, 64])
+def test_criteria_outside_the_corrected_range(lc, orc, wl, dev, n):
+    """Columns scaled so far down (with a large entry kept in each row) that
+    their criteria need the division, rows above the reciprocal's range, and
+    non-finite entries met inside a panel."""
+    base = wl.gaussian_np(8, n, seed=4000 + n)
+    A = base.copy()
+    A[0][:, : n // 2] *= 2.0 ** -900
+    A[1][:, 1::3] *= 2.0 ** -1000
+    A[2] *= 2.0 ** 1000
+    A[3][::2] *= 2.0 ** 970
+    A[4][:, 6] *= 2.0 ** -1040
+    A[5][n // 3, n - 2] = np.inf
+    A[6][n // 2, 9] = complex(np.nan, 1.0)
+    A[7][:, 3] = 0.0
+    A[7][n - 1, 3] = 2.0 ** -950
+    check(lc, orc, dev, A)
