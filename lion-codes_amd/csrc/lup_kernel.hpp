@@ -1079,15 +1079,11 @@ constexpr ShapeLC candidate_shape(int n, int idx) {
     return c[idx];
   }
   if (n <= 24) {
-    constexpr ShapeLC c[] = {{32, 4, 2, false}, {16, 2, 2, false}, {32, 2, 2, false}, {32, 4, 3, true}};
+    constexpr ShapeLC c[] = {{32, 4, 2, false}, {16, 2, 2, false}, {32, 2, 2, false}, {32, 4, 2, true}};
     return c[idx];
   }
   if (n <= 32) {
     constexpr ShapeLC c[] = {{32, 4, 2, true}, {32, 2, 2, false}, {32, 1, 2, false}, none};
-    return c[idx];
-  }
-  if (n <= 40) {
-    constexpr ShapeLC c[] = {{64, 4, 2, true}, {64, 4, 3, true}, none, none};
     return c[idx];
   }
   if (n <= 48) {
