@@ -1056,11 +1056,11 @@ __global__ void __launch_bounds__(64 * WPB, OCC) lup_det_kernel(BatchArgs args) 
 // each row over lane-columns.  The panel kernel (lup_panel.hpp) takes a fixed
 // lane per row of its panel, so it loses where rows are few (n = 17: 2.57
 // against 1.97, n = 20: 2.92 against 2.45), wins at odd n in between (n = 23:
-// 3.67 against 4.77) and from n = 25 on (n = 32: 6.8 against 7.8, n = 48: 19.8
-// against 26.0, n = 64: 50 against 81), so from n = 33 it is the only one.
-// Two waves per SIMD hide its serial steps; above n = 48 that costs spills of
-// the first panels' slots, which still pays at n = 56 (35.1 against 38.6) and
-// no longer at n = 64 (52.8 against 49.4).
+// 3.65 against 4.77) and from n = 25 on (n = 32: 6.6 against 7.8, n = 48: 18.5
+// against 26.0, n = 64: 49 against 81), so from n = 33 it is the only one.
+// Two waves per SIMD hide its serial steps; above n = 52 that costs spills of
+// the first panels' slots, which still pays at n = 56 (348 us for 10699
+// matrices against 380) and no longer from n = 57 on (446 against 422).
 struct ShapeLC {
   int lanes;
   int lane_cols;

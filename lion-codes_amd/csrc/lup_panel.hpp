@@ -57,8 +57,36 @@ constexpr int panel_lds(int n) {
   return g * (panel_area(g) + panel_pivot_area(n)) + (g > 1 ? g * 6 : 0) + 16;
 }
 
+// Row slots a matrix still needs when panel p is searched (p = 0: all).  Once
+// the rows left fit in one slot less and at least kMinPanelsLeft panels
+// follow, the rows of the last slot move into the places of finished rows:
+// their trailing columns through the panel's LDS area (one slot is written,
+// only the places that take a row read), the row's state by ds_bpermute.  All
+// later panels then update, write and read one slot less.  Measured with and
+// without, ns per determinant: n = 32 6.55 / 6.88, n = 40 13.4 / 14.6, n = 48
+// 18.5 / 19.7, n = 52 24.1 / 30.8 (one slot less after the first panel, and so
+// no spills at two waves per SIMD), n = 64 48.7 / 50.4.
+constexpr int kMinPanelsLeft = 2;
+constexpr int panel_slots(int n, int p) {
+  const int rg = 16 / panel_groups(n), c = (n + 3) / 4;
+  int r = (n + rg - 1) / rg;
+  for (int q = 0; q < p; ++q)
+    if (r > 1 && n - 4 * (q + 1) <= (r - 1) * rg && c - 1 - q >= kMinPanelsLeft) --r;
+  return r;
+}
+
+struct PanelSlots {
+  int at[17];
+};
+constexpr PanelSlots panel_slot_table(int n) {
+  PanelSlots t{};
+  for (int p = 0; p <= 16; ++p) t.at[p] = panel_slots(n, p);
+  return t;
+}
+
 template <int N, int G>
 struct PanelTile {
+  static constexpr PanelSlots slots = panel_slot_table(N);
   static_assert(G == 1 || G == 2, "matrices per wave");
   static constexpr int L = 64 / G;             // panel layout: lanes (rows) per matrix
   static constexpr int RG = 16 / G;            // tile layout: lane-rows per matrix
@@ -103,6 +131,24 @@ constexpr uint64_t group_lanes(uint64_t bits) {
   uint64_t r = 0;
   for (int g = 0; g < G; ++g) r |= bits << (g * (64 / G));
   return r;
+}
+
+// Bits of `m` below this lane, in its group.
+template <int G>
+__device__ __forceinline__ int group_rank(uint64_t m, int lane) {
+  const int lo = __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0);
+  if constexpr (G == 1) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), lo);
+  } else {
+    const int hi = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), 0);
+    return lane < 32 ? lo : hi;
+  }
+}
+
+__device__ __forceinline__ double bpermute_d(int addr, double v) {
+  const int lo = __builtin_amdgcn_ds_bpermute(addr, __double2loint(v));
+  const int hi = __builtin_amdgcn_ds_bpermute(addr, __double2hiint(v));
+  return __hiloint2double(hi, lo);
 }
 
 // RN(1/d) for d in [0.25, 2); any finite value for d == 0.
@@ -333,6 +379,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
   for (int p = 0; p < C; ++p) {
     constexpr int W = 4;
     const int nb = N - 4 * p < W ? N - 4 * p : W;
+    const int R1 = T::slots.at[p], R2 = T::slots.at[p + 1];
     const bool trail = p + 1 < C;
     double px[W], py[W];
     int pa[W];  // LDS row of each pivot (double2)
@@ -409,7 +456,8 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
         pjv[lane] = pj;
         wave_lds_sync();
 #pragma unroll
-        for (int t = 0; t < R; ++t) tj[t] = pjv[gt * L + rb + RG * t];
+        for (int t = 0; t < R; ++t)
+          if (t < R1) tj[t] = pjv[gt * L + rb + RG * t];
       }
       if (trail && j == W - 1) {
         // raw pivot rows to LDS
@@ -419,6 +467,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
         const int pt = select_group<G>(pl, gt);
 #pragma unroll
         for (int t = 0; t < R; ++t) {
+          if (t >= R1) continue;
           const int q = rb + RG * t == pt ? j : tj[t];
           if (q >= 0) {
             double2* dst = ub + gt * GS + q * US + jc;
@@ -496,11 +545,88 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
     if (!trail) continue;
 
     wave_lds_sync();
+    int sa[R], st[R];  // place each row slot's row comes from (operand and tile lanes)
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      sa[t] = rba + RG * t;
+      st[t] = rb + RG * t;
+    }
+    if (R2 < R1) {
+      // finished places below R2 row slots take the active rows above, in order
+      const int low = R2 * RG;
+      const uint64_t lowm = group_lanes<G>((1ull << low) - 1ull);
+      const uint64_t up = am & ~lowm, dead = ~am & lowm;
+      const int ru = group_rank<G>(up, lane), rd = group_rank<G>(dead, lane);
+      int nu[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) nu[g] = __builtin_popcountll(group_bits<G>(up, g));
+      if (__builtin_amdgcn_inverse_ballot_w64(up)) pjv[gp * L + ru] = row;
+      wave_lds_sync();
+      const uint64_t take =
+          dead & __builtin_amdgcn_ballot_w64(rd < select_group<G>(nu, gp));
+      int from = row;
+      if (__builtin_amdgcn_inverse_ballot_w64(take)) from = pjv[gp * L + rd];
+      wave_lds_sync();
+      pjv[lane] = from;
+      const int fl = (gp * L + from) * 4;
+      pos = __builtin_amdgcn_ds_bpermute(fl, pos);
+      if constexpr (POLICY == POLICY_CROUT_REF) {
+        sc = bpermute_d(fl, sc);
+        rs = bpermute_d(fl, rs);
+      }
+      am = (am & lowm) | take;
+      wave_lds_sync();
+#pragma unroll
+      for (int t = 0; t < R; ++t) {
+        if (t >= R2) continue;
+        sa[t] = pjv[gt * L + rba + RG * t];
+        st[t] = pjv[gt * L + rb + RG * t];
+      }
+    }
 #pragma unroll
     for (int t = 0; t < R; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        Ax[t][h] = pd[(gt * PG + (rba + RG * t) * PS) * 2 + 4 * h + ti];
+        if (t < R2) Ax[t][h] = pd[(gt * PG + sa[t] * PS) * 2 + 4 * h + ti];
+    if (R2 < R1) {
+      // the moved rows' trailing columns, through the panel's area
+      wave_lds_sync();
+      constexpr int SW = 4;  // column slots a round moves
+      static_assert(RG * (4 * SW + 1) <= L * PS, "staging area");
+      double2* stage = pan + gt * PG;
+#pragma unroll
+      for (int s0 = 0; s0 < C; s0 += SW) {
+        if (s0 + SW <= p + 1) continue;
+#pragma unroll
+        for (int c = 0; c < SW; ++c)
+          if (s0 + c > p && s0 + c < C)
+            stage[rb * (4 * SW + 1) + 4 * c + jc] =
+                make_double2(ax[R1 - 1][s0 + c], ay[R1 - 1][s0 + c]);
+        wave_lds_sync();
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+          if (t >= R2) continue;
+          // by value, so that no address into the tile is ever selected
+          double2 v[SW];
+#pragma unroll
+          for (int c = 0; c < SW; ++c)
+            if (s0 + c > p && s0 + c < C) v[c] = make_double2(ax[t][s0 + c], ay[t][s0 + c]);
+          if (st[t] >= R2 * RG) {
+            const double2* row_t = stage + (st[t] - R2 * RG) * (4 * SW + 1) + jc;
+#pragma unroll
+            for (int c = 0; c < SW; ++c)
+              if (s0 + c > p && s0 + c < C) v[c] = row_t[4 * c];
+          }
+#pragma unroll
+          for (int c = 0; c < SW; ++c)
+            if (s0 + c > p && s0 + c < C) {
+              ax[t][s0 + c] = v[c].x;
+              ay[t][s0 + c] = v[c].y;
+            }
+        }
+        wave_lds_sync();
+      }
+    }
     // trailing update, the next panel first
 #pragma unroll
     for (int s = 0; s < C; ++s) {
@@ -515,13 +641,14 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int t = 0; t < R; ++t) {
+          if (t >= R2) continue;
           ax[t][s] = mfma_4x4x4(Ax[t][h], Bx[h], ax[t][s]);
           ay[t][s] = mfma_4x4x4(Ax[t][h], By[h], ay[t][s]);
         }
       if (s == p + 1) {
 #pragma unroll
         for (int t = 0; t < R; ++t)
-          tile[RG * t * PS] = make_double2(ax[t][s], ay[t][s]);
+          if (t < R2) tile[RG * t * PS] = make_double2(ax[t][s], ay[t][s]);
         wave_lds_sync();
       }
     }
