@@ -222,31 +222,27 @@ int32_t lufqhe_fqhe_build(const void *d_z, int64_t count, int32_t n,
  * per-bucket offset / output-slot tables (16 B per matrix, allocated here,
  * freed by lufqhe_mixed_plan_destroy) and creates `nstreams` streams for the
  * buckets, assigned largest-cost-first.  Fused arithmetic, the given pivot
- * policy, the launch shape selected for each n.
+ * policy.
  *
  * lufqhe_mixed_execute writes det outputs (as lufqhe_det_batched) at each
  * matrix's own index m.  source LUFQHE_SOURCE_MATRIX reads matrix m at
  * d_A + offs[m]; LUFQHE_SOURCE_FQHE reads n[m] particle positions there and
  * builds the FQHE matrix on the device (as lufqhe_fqhe_det).  Modes:
- *   LUFQHE_MIXED_GRAPH    the bucket launches forked over the plan streams,
+ *   LUFQHE_MIXED_GRAPH    one launch per size with enough matrices to fill
+ *                         the device (with the launch shape selected for that
+ *                         size at capture time) and one per class (n <= 8,
+ *                         9..16, 17..32, 33..56, 57..64) of the other sizes
+ *                         (with fixed shapes), forked over the plan streams,
  *                         captured into one hipGraph on the first call for a
  *                         given set of pointers and source (instantiation
- *                         allocates) and replayed after -- with the launch
- *                         shapes selected at capture time; `stream` must not
+ *                         allocates) and replayed after; `stream` must not
  *                         be the legacy default stream (capture is not
  *                         allowed there);
  *   LUFQHE_MIXED_STREAMS  the same forked launches, issued directly;
- *   LUFQHE_MIXED_PLAIN    one launch per size, one after another on `stream`;
- *   LUFQHE_MIXED_PERSISTENT  one persistent kernel per size class (n <= 16,
- *                         17..32, 33..48, 49..57, 58..64) instead of one
- *                         launch per bucket: resident waves drain the class's
- *                         buckets, largest n first, from a device work
- *                         counter that a kernel at the head of the graph
- *                         zeroes.  Captured and replayed like GRAPH (the
- *                         per-bucket arguments are written to device memory,
- *                         synchronously, when the pointers change).  Fused
- *                         arithmetic with either policy; a plan with 2^31 or
- *                         more tasks in one class refuses this mode
+ *   LUFQHE_MIXED_PLAIN    one launch per size with the shape selected for it,
+ *                         one after another on `stream`;
+ *   LUFQHE_MIXED_PERSISTENT  the same as GRAPH; a plan with 2^31 or more
+ *                         workgroups of one size refuses it
  *                         (LUFQHE_ERROR_UNSUPPORTED).
  * A plan is not re-entrant: one execute at a time per plan, on the device
  * that was current when it was created (else LUFQHE_ERROR_INVALID_VALUE). */

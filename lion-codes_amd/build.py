@@ -10,7 +10,7 @@
 
 Kernels are instantiated per (variant, n); ``lup_inst.hip`` is compiled once
 per (variant, shard) so the fully unrolled kernels compile in parallel, and
-``lup_persist_inst.hip`` once per (fused variant, size class).
+``lup_class_inst.hip`` once per (fused variant, size class).
 """
 from __future__ import annotations
 
@@ -32,8 +32,8 @@ ORACLE_LIB = ORACLE_DIR / "liblufqhe_oracle.so"
 ARCH = "gfx950"
 N_VARIANTS = 3
 N_SHARDS = 8
-N_PERSIST_VARIANTS = 2  # persistent mixed-size kernels: fused CROUT_REF and ABS
-N_PERSIST_CLASSES = 5   # size classes of lup_persistent.hpp
+N_CLASS_VARIANTS = 2  # class kernels: fused CROUT_REF and ABS
+N_CLASSES = 5         # size classes of lup_class.hpp
 
 HIP_FLAGS = [
     f"--offload-arch={ARCH}",
@@ -80,13 +80,13 @@ def _compile_jobs() -> list[tuple[Path, list[str], list[Path]]]:
     # the kernel instantiation units include only the kernel headers
     kern_hdrs = sorted(CSRC.glob("*.hpp"))
     jobs = []
-    # the persistent class kernels are the longest single compiles: first
-    for v in range(N_PERSIST_VARIANTS):
-        for c in range(N_PERSIST_CLASSES):
-            obj = BUILD / f"lup_persist_v{v}_c{c}.o"
+    # the class kernels of the large sizes are the longest single compiles: first
+    for c in reversed(range(N_CLASSES)):
+        for v in range(N_CLASS_VARIANTS):
+            obj = BUILD / f"lup_class_v{v}_c{c}.o"
             defs = [f"-DLUFQHE_VARIANT={v}", f"-DLUFQHE_CLASS={c}"]
-            jobs.append((obj, defs + ["-c", str(CSRC / "lup_persist_inst.hip")],
-                         kern_hdrs + [CSRC / "lup_persist_inst.hip"]))
+            jobs.append((obj, defs + ["-c", str(CSRC / "lup_class_inst.hip")],
+                         kern_hdrs + [CSRC / "lup_class_inst.hip"]))
     for v in range(N_VARIANTS):
         for s in range(N_SHARDS):
             obj = BUILD / f"lup_inst_v{v}_s{s}.o"
@@ -94,7 +94,7 @@ def _compile_jobs() -> list[tuple[Path, list[str], list[Path]]]:
             jobs.append((obj, defs + ["-c", str(CSRC / "lup_inst.hip")],
                          kern_hdrs + [CSRC / "lup_inst.hip"]))
     for src in sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.cpp")):
-        if src.name in ("lup_inst.hip", "lup_persist_inst.hip"):
+        if src.name in ("lup_inst.hip", "lup_class_inst.hip"):
             continue
         obj = BUILD / (src.stem + ".o")
         lang = ["-x", "hip"] if src.suffix == ".hip" else []

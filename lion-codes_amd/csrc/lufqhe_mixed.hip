@@ -3,22 +3,24 @@
 // The reference handles one matrix size per run (RunInfo, LU-fqhe/src/
 // RunInfo.cpp:46-78); a batch of mixed sizes there means one CALL per size
 // on repacked uniform batches.  Here a plan buckets the batch by n once:
-//   * per-bucket tables of element offsets and output slots live on the
-//     device (one allocation, made when the plan is created);
-//   * each bucket is one launch of that n's tuned kernel with indexed
-//     addressing (BatchArgs::offs / out_idx), so nothing is repacked;
-//   * buckets are spread over the plan's streams largest-cost-first
+//   * tables of element offsets and output slots sorted by n live on the
+//     device (one allocation, made when the plan is created), so nothing is
+//     repacked;
+//   * a size with enough matrices to fill the device is one launch of its own
+//     kernel; the other sizes of a class share one launch of the class's
+//     kernel (lup_class.hpp);
+//   * the launches are spread over the plan's streams largest-cost-first
 //     (longest-processing-time assignment on F(n) * count) and forked from /
-//     joined to the caller's stream with events, so small-n buckets run
-//     beside the big ones instead of after them;
+//     joined to the caller's stream with events, so the small ones run beside
+//     the large ones instead of after them;
 //   * the whole fork/launch/join sequence is captured once into a hipGraph
-//     and replayed: one graph launch per batch.
-// Mode PERSISTENT replaces the per-bucket launches by one persistent kernel
-// per size class (lup_persistent.hpp): the buckets of a class form one
-// device work queue, drained largest n first by resident waves; the queue
-// counters are zeroed by a small kernel at the head of the captured graph.
-// Mode PLAIN runs the same kernels one size after another on the caller's
-// stream: the uniform-launch-per-size form it is compared with.
+//     and replayed: one graph launch per batch.  PERSISTENT is the same
+//     sequence.
+// A launch per size leaves wave slots empty when its bucket is small, and each
+// waited for the one before it on its stream: 32768 FQHE matrices of 31 sizes
+// took 298 us that way and take 239, 2675 matrices of 24 sizes 353 and 130.
+// Mode PLAIN runs each size's own kernel one after another on the caller's
+// stream: the uniform-launch-per-size form the others are compared with.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -53,36 +55,21 @@ struct lufqhe_mixed_plan {
   hipStream_t streams[LUFQHE_MIXED_MAX_STREAMS] = {};
   hipEvent_t fork = nullptr;
   hipEvent_t join[LUFQHE_MIXED_MAX_STREAMS] = {};
-  // recorded after every persistent replay: the per-bucket arguments those
-  // replays read are rewritten only once it has completed
-  hipEvent_t replayed = nullptr;
-  bool replay_pending = false;
-  // persistent mode: per class, its buckets' queue and launch size
-  struct PClass {
-    int cls = 0;
-    int64_t first = 0;  // first bucket of the class in the device arrays
-    int32_t nbuckets = 0;
-    int64_t total_tasks = 0;
-    int64_t blocks = 0;
+  bool used[LUFQHE_MIXED_MAX_STREAMS] = {};  // streams a launch is assigned to
+  // one launch: a bucket by its size's own kernel, or a class of small buckets
+  struct Launch {
+    int bucket = -1;  // else `group`
+    ClassBatch group;
     double cost = 0.0;
     int stream = 0;
   };
-  std::vector<PClass> pclasses;           // in launch order
-  std::vector<BatchArgs> h_bargs;         // per bucket, in class order
-  std::vector<int32_t> h_bucket_index;    // bargs slot -> plan bucket
-  void* d_persist = nullptr;              // PersistBucket[] | BatchArgs[] | counters
-  PersistBucket* d_pbuckets = nullptr;
-  BatchArgs* d_bargs = nullptr;
-  uint32_t* d_counters = nullptr;
-  const void* p_A = nullptr;              // pointers d_bargs holds
-  int p_src = -1;
-  DetOut p_out{};
+  std::vector<Launch> launches;  // in launch order
+  bool too_large = false;        // a bucket of 2^31 or more workgroups
   // captured graph and what it was captured for
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   const void* g_A = nullptr;
   int g_src = 0;
-  int g_mode = -1;
   DetOut g_out{};
 
   ~lufqhe_mixed_plan() {
@@ -93,9 +80,7 @@ struct lufqhe_mixed_plan {
       if (streams[s]) (void)hipStreamDestroy(streams[s]);
     }
     if (fork) (void)hipEventDestroy(fork);
-    if (replayed) (void)hipEventDestroy(replayed);
     if (d_tables) (void)hipFree(d_tables);
-    if (d_persist) (void)hipFree(d_persist);
   }
 };
 
@@ -121,17 +106,32 @@ hipError_t launch_bucket(const lufqhe_mixed_plan& p, const lufqhe_mixed_plan::Bu
   return e.launch(args, plain_blocks(e, b.count), stream);
 }
 
-// Fork from `stream`, one launch sequence per plan stream, join back.
+BatchArgs class_args(const lufqhe_mixed_plan& p, const void* d_A, int src, const DetOut& out) {
+  BatchArgs args{};
+  args.A = static_cast<const double2*>(d_A);
+  args.offs = p.d_tables;
+  args.out_idx = p.d_tables + p.count;
+  args.src = src;
+  args.out = out;
+  return args;
+}
+
+// Fork from `stream`, the launches on the plan's streams, join back.
 hipError_t issue_forked(const lufqhe_mixed_plan& p, const void* d_A, int src,
                         const DetOut& out, hipStream_t stream) {
+  const BatchArgs args = class_args(p, d_A, src, out);
+  auto launch = [&](const lufqhe_mixed_plan::Launch& l, hipStream_t s) {
+    return l.bucket >= 0 ? launch_bucket(p, p.buckets[l.bucket], d_A, src, out, s)
+                         : l.group.launch(p.variant, args, s);
+  };
+  if (p.launches.size() == 1) return launch(p.launches[0], stream);
   hipError_t err = hipEventRecord(p.fork, stream);
   for (int s = 0; s < p.nstreams && err == hipSuccess; ++s)
-    err = hipStreamWaitEvent(p.streams[s], p.fork, 0);
-  for (const auto& b : p.buckets) {
-    if (err != hipSuccess) break;
-    err = launch_bucket(p, b, d_A, src, out, p.streams[b.stream]);
-  }
+    if (p.used[s]) err = hipStreamWaitEvent(p.streams[s], p.fork, 0);
+  for (const auto& l : p.launches)
+    if (err == hipSuccess) err = launch(l, p.streams[l.stream]);
   for (int s = 0; s < p.nstreams && err == hipSuccess; ++s) {
+    if (!p.used[s]) continue;
     err = hipEventRecord(p.join[s], p.streams[s]);
     if (err == hipSuccess) err = hipStreamWaitEvent(stream, p.join[s], 0);
   }
@@ -143,126 +143,52 @@ bool same_out(const DetOut& a, const DetOut& b) {
          a.info == b.info && a.piv == b.piv;
 }
 
-__global__ void __launch_bounds__(64) persist_reset_kernel(uint32_t* __restrict__ counters, int n) {
-  if ((int)threadIdx.x < n) counters[threadIdx.x] = 0u;
-}
-
-// The class queues of a plan: buckets grouped by size class, largest n
-// first within a class, with their task ranges; classes ordered and spread
-// over the plan streams by cost.  Device arrays are allocated here; the
-// per-bucket launch arguments are written when the pointers are known.
-hipError_t build_persistent(lufqhe_mixed_plan& p) {
-  if (p.variant >= kPersistVariants) return hipSuccess;  // no persistent kernels for it
+// The plan's launches.  A bucket that fills the device's wave slots runs its
+// size's own kernel; the others of a class share one launch, largest n first.
+// Longest-processing-time assignment to the plan's streams.
+hipError_t build_launches(lufqhe_mixed_plan& p) {
   int cus = 0;
-  hipError_t err = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p.device);
+  const hipError_t err =
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p.device);
   if (err != hipSuccess) return err;
-  std::vector<PersistBucket> hb;
-  for (int c = 0; c < kPersistClasses; ++c) {
-    std::vector<int> idx;
-    for (int i = 0; i < (int)p.buckets.size(); ++i)
-      if (persist_class(p.buckets[i].n) == c) idx.push_back(i);
-    if (idx.empty()) continue;
-    std::sort(idx.begin(), idx.end(), [&](int a, int b) { return p.buckets[a].n > p.buckets[b].n; });
-    lufqhe_mixed_plan::PClass pc;
-    pc.cls = c;
-    pc.first = (int64_t)hb.size();
-    pc.nbuckets = (int32_t)idx.size();
-    for (int i : idx) {
-      const auto& b = p.buckets[i];
-      const int g = persist_group(b.n);
-      hb.push_back(PersistBucket{b.n, 0, pc.total_tasks});
-      p.h_bucket_index.push_back(i);
-      pc.total_tasks += (b.count + g - 1) / g;
-      pc.cost += b.cost;
+  std::vector<int> order(p.buckets.size());
+  for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
+  std::sort(order.begin(), order.end(),
+            [&](int a, int b) { return p.buckets[a].n > p.buckets[b].n; });
+  int open[kClasses];  // the class's shared launch
+  std::fill(open, open + kClasses, -1);
+  for (int i : order) {
+    const auto& b = p.buckets[i];
+    const int64_t blocks = plain_blocks(entry_for(p.variant, b.n), b.count);
+    p.too_large = p.too_large || blocks > INT32_MAX;
+    if (fills_device(blocks, cus)) {
+      p.launches.emplace_back();
+      p.launches.back().bucket = i;
+      p.launches.back().cost = b.cost;
+      continue;
     }
-    // the class counter is 32-bit and every wave adds one past the end: a
-    // class too large for it gets no persistent launch (the mode is refused)
-    if (pc.total_tasks >= (int64_t{1} << 31)) {
-      p.pclasses.clear();
-      p.h_bucket_index.clear();
-      return hipSuccess;
+    int& o = open[size_class(b.n)];
+    if (o < 0) {
+      o = (int)p.launches.size();
+      p.launches.emplace_back();
+      p.launches.back().group.cls = size_class(b.n);
     }
-    const PersistEntry& e = g_persist[p.variant][c];
-    if (!e.launch) return hipErrorInvalidDeviceFunction;
-    int per_cu = 0;
-    err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, e.kernel, 64, 0);
-    if (err != hipSuccess) return err;
-    pc.blocks = std::min<int64_t>(pc.total_tasks, (int64_t)std::max(1, per_cu) * cus);
-    p.pclasses.push_back(pc);
+    if (!p.launches[o].group.add(b.n, b.start, b.count)) return hipErrorInvalidValue;
+    p.launches[o].cost += b.cost;
   }
-  std::sort(p.pclasses.begin(), p.pclasses.end(),
-            [](const auto& a, const auto& b) { return a.cost > b.cost; });
+  std::stable_sort(p.launches.begin(), p.launches.end(),
+                   [](const auto& a, const auto& b) { return a.cost > b.cost; });
   std::vector<double> load(p.nstreams, 0.0);
-  for (auto& pc : p.pclasses) {
-    const int s = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    pc.stream = s;
-    load[s] += pc.cost;
+  for (auto& l : p.launches) {
+    l.stream = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    load[l.stream] += l.cost;
+    p.used[l.stream] = true;
+    if (l.bucket >= 0) p.buckets[l.bucket].stream = l.stream;
+    for (int j = 0; j < l.group.ca.nbuckets; ++j)
+      for (auto& b : p.buckets)
+        if (b.n == l.group.ca.n[j]) b.stream = l.stream;
   }
-  p.h_bargs.assign(hb.size(), BatchArgs{});
-  const size_t nb = hb.size();
-  const size_t o_bargs = (nb * sizeof(PersistBucket) + 255) & ~(size_t)255;
-  const size_t o_cnt = (o_bargs + nb * sizeof(BatchArgs) + 255) & ~(size_t)255;
-  if (nb == 0) return hipSuccess;
-  err = hipMalloc(&p.d_persist, o_cnt + kPersistClasses * sizeof(uint32_t));
-  if (err != hipSuccess) return err;
-  char* base = static_cast<char*>(p.d_persist);
-  p.d_pbuckets = reinterpret_cast<PersistBucket*>(base);
-  p.d_bargs = reinterpret_cast<BatchArgs*>(base + o_bargs);
-  p.d_counters = reinterpret_cast<uint32_t*>(base + o_cnt);
-  return hipMemcpy(p.d_pbuckets, hb.data(), nb * sizeof(PersistBucket), hipMemcpyHostToDevice);
-}
-
-// Per-bucket launch arguments for these pointers (synchronous, outside any
-// capture; the caller has drained `stream`, the only user of the old ones).
-hipError_t write_persistent_args(lufqhe_mixed_plan& p, const void* d_A, int src,
-                                 const DetOut& out) {
-  for (size_t j = 0; j < p.h_bargs.size(); ++j) {
-    const auto& b = p.buckets[p.h_bucket_index[j]];
-    BatchArgs& a = p.h_bargs[j];
-    a = BatchArgs{};
-    a.A = static_cast<const double2*>(d_A);
-    a.count = b.count;
-    a.ld = b.n;
-    a.stride = 0;
-    a.offs = p.d_tables + b.start;
-    a.out_idx = p.d_tables + p.count + b.start;
-    a.piv_stride = 0;
-    a.src = src;
-    a.out = out;
-  }
-  hipError_t err = hipMemcpy(p.d_bargs, p.h_bargs.data(), p.h_bargs.size() * sizeof(BatchArgs),
-                             hipMemcpyHostToDevice);
-  if (err == hipSuccess) {
-    p.p_A = d_A;
-    p.p_src = src;
-    p.p_out = out;
-  }
-  return err;
-}
-
-// Reset the class counters, fork, one persistent launch per class, join.
-hipError_t issue_persistent(const lufqhe_mixed_plan& p, hipStream_t stream) {
-  hipLaunchKernelGGL(persist_reset_kernel, dim3(1), dim3(64), 0, stream, p.d_counters,
-                     kPersistClasses);
-  hipError_t err = hipGetLastError();
-  if (err == hipSuccess) err = hipEventRecord(p.fork, stream);
-  for (int s = 0; s < p.nstreams && err == hipSuccess; ++s)
-    err = hipStreamWaitEvent(p.streams[s], p.fork, 0);
-  for (const auto& pc : p.pclasses) {
-    if (err != hipSuccess) break;
-    PersistArgs pa{};
-    pa.buckets = p.d_pbuckets + pc.first;
-    pa.bargs = p.d_bargs + pc.first;
-    pa.nbuckets = pc.nbuckets;
-    pa.counter = p.d_counters + pc.cls;
-    pa.total_tasks = pc.total_tasks;
-    err = g_persist[p.variant][pc.cls].launch(pa, pc.blocks, p.streams[pc.stream]);
-  }
-  for (int s = 0; s < p.nstreams && err == hipSuccess; ++s) {
-    err = hipEventRecord(p.join[s], p.streams[s]);
-    if (err == hipSuccess) err = hipStreamWaitEvent(stream, p.join[s], 0);
-  }
-  return err;
+  return hipSuccess;
 }
 
 }  // namespace
@@ -307,22 +233,15 @@ int32_t lufqhe_mixed_plan_create(const int32_t* h_n, const int64_t* h_offs, int6
     b.cost = det_flops(n) * (double)per_n[n] + 16.0 * n * n * per_n[n];
     p->buckets.push_back(b);
   }
-  // longest-processing-time assignment, largest first within each stream
+  // reported in launch order, largest cost first
   std::sort(p->buckets.begin(), p->buckets.end(),
             [](const auto& a, const auto& b) { return a.cost > b.cost; });
-  std::vector<double> load(nstreams, 0.0);
-  for (auto& b : p->buckets) {
-    const int s = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    b.stream = s;
-    load[s] += b.cost;
-  }
 
   if (err == hipSuccess && count > 0) err = hipMalloc(&p->d_tables, tables.size() * sizeof(int64_t));
   if (err == hipSuccess && count > 0)
     err = hipMemcpy(p->d_tables, tables.data(), tables.size() * sizeof(int64_t),
                     hipMemcpyHostToDevice);
   if (err == hipSuccess) err = hipEventCreateWithFlags(&p->fork, hipEventDisableTiming);
-  if (err == hipSuccess) err = hipEventCreateWithFlags(&p->replayed, hipEventDisableTiming);
   for (int s = 0; s < nstreams && err == hipSuccess; ++s) {
     err = hipStreamCreateWithFlags(&p->streams[s], hipStreamNonBlocking);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&p->join[s], hipEventDisableTiming);
@@ -336,7 +255,7 @@ int32_t lufqhe_mixed_plan_create(const int32_t* h_n, const int64_t* h_offs, int6
       delete p;
       return LUFQHE_ERROR_NOT_BUILT;
     }
-  err = build_persistent(*p);
+  err = build_launches(*p);
   if (err != hipSuccess) {
     delete p;
     return hip_fail(err);
@@ -390,26 +309,16 @@ int32_t lufqhe_mixed_execute(lufqhe_mixed_plan* plan, const void* d_A, void* d_m
     err = issue_forked(*plan, d_A, src, out, stream);
   } else if (mode == LUFQHE_MIXED_GRAPH || mode == LUFQHE_MIXED_PERSISTENT) {
     if (stream == nullptr) return LUFQHE_ERROR_INVALID_VALUE;  // no capture on stream 0
-    const bool persistent = mode == LUFQHE_MIXED_PERSISTENT;
-    if (persistent && (plan->variant >= kPersistVariants || plan->pclasses.empty()))
-      return LUFQHE_ERROR_UNSUPPORTED;
-    if (!plan->exec || plan->g_mode != mode || plan->g_A != d_A || plan->g_src != src ||
+    if (mode == LUFQHE_MIXED_PERSISTENT && plan->too_large) return LUFQHE_ERROR_UNSUPPORTED;
+    if (!plan->exec || plan->g_A != d_A || plan->g_src != src ||
         !same_out(plan->g_out, out)) {
       if (plan->exec) (void)hipGraphExecDestroy(plan->exec);
       if (plan->graph) (void)hipGraphDestroy(plan->graph);
       plan->exec = nullptr;
       plan->graph = nullptr;
-      plan->g_mode = -1;
-      if (persistent && (plan->p_A != d_A || plan->p_src != src || !same_out(plan->p_out, out))) {
-        // earlier replays, on whatever stream, may still read the old
-        // arguments: wait for the last one
-        if (plan->replay_pending) err = hipEventSynchronize(plan->replayed);
-        if (err == hipSuccess) err = write_persistent_args(*plan, d_A, src, out);
-      }
       if (err == hipSuccess) err = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
       if (err == hipSuccess) {
-        const hipError_t e2 = persistent ? issue_persistent(*plan, stream)
-                                         : issue_forked(*plan, d_A, src, out, stream);
+        const hipError_t e2 = issue_forked(*plan, d_A, src, out, stream);
         err = hipStreamEndCapture(stream, &plan->graph);
         if (e2 != hipSuccess) err = e2;
       }
@@ -417,15 +326,10 @@ int32_t lufqhe_mixed_execute(lufqhe_mixed_plan* plan, const void* d_A, void* d_m
       if (err == hipSuccess) {
         plan->g_A = d_A;
         plan->g_src = src;
-        plan->g_mode = mode;
         plan->g_out = out;
       }
     }
     if (err == hipSuccess) err = hipGraphLaunch(plan->exec, stream);
-    if (err == hipSuccess && persistent) {
-      err = hipEventRecord(plan->replayed, stream);
-      plan->replay_pending = err == hipSuccess;
-    }
   } else {
     return LUFQHE_ERROR_INVALID_VALUE;
   }

@@ -16,8 +16,8 @@
 //    are still running (continuous batching);
 //  * each batch is: one prepare kernel (moves particles into per-request
 //    configuration slots, commits accepted configurations, expands per-term
-//    index tables), one determinant launch per n bucket with the FQHE matrix
-//    built in the kernel's load phase, one per-request sum kernel, one small
+//    index tables), determinant launches (one per size that fills the device, one per
+//    class of the others) with the FQHE matrix built in the load phase, one per-request sum kernel, one small
 //    device-to-host copy of the sums;
 //  * on completion the host applies the Metropolis rule
 //    |psi'|^2 >= u |psi|^2 (u from the request's own random stream).
@@ -161,6 +161,7 @@ static_assert(sizeof(ReqDesc) == 64, "ReqDesc layout");
 // ---------------------------------------------------------------- server
 struct lufqhe_server {
   int device = 0;
+  int cus = 0;  // compute units of the device
   int variant = 0;
   int walkers = 0;
   int perms = 0;
@@ -335,20 +336,34 @@ struct Run {
                          b.d_out_idx);
       err = hipGetLastError();
     }
-    for (int n = 1; n <= kMaxN && err == hipSuccess; ++n) {
-      if (!per_n[n]) continue;
-      const KernelEntry& e = entry_for(s->variant, n);
-      BatchArgs a{};
-      a.A = d_slot_z;
-      a.count = per_n[n];
-      a.ld = n;
-      a.offs = b.d_offs + start[n];
-      a.out_idx = b.d_out_idx + start[n];
-      a.row_perm = s->d_perm;
-      a.perm_offs = b.d_perm_offs + start[n];
-      a.src = SRC_FQHE;
-      a.out = DetOut{b.d_mant, b.d_exp, nullptr, nullptr, nullptr, nullptr};
-      err = e.launch(a, plain_blocks(e, per_n[n]), b.stream);
+    BatchArgs a{};
+    a.A = d_slot_z;
+    a.offs = b.d_offs;
+    a.out_idx = b.d_out_idx;
+    a.row_perm = s->d_perm;
+    a.perm_offs = b.d_perm_offs;
+    a.src = SRC_FQHE;
+    a.out = DetOut{b.d_mant, b.d_exp, nullptr, nullptr, nullptr, nullptr};
+    for (int c = kClasses - 1; c >= 0 && err == hipSuccess; --c) {
+      ClassBatch cb;
+      cb.cls = c;
+      for (int n = kClassHi[c]; n >= kClassLo[c] && err == hipSuccess; --n) {
+        if (!per_n[n]) continue;
+        const KernelEntry& e = entry_for(s->variant, n);
+        const int64_t blocks = plain_blocks(e, per_n[n]);
+        if (fills_device(blocks, s->cus)) {
+          BatchArgs one = a;
+          one.count = per_n[n];
+          one.ld = n;
+          one.offs += start[n];
+          one.out_idx += start[n];
+          one.perm_offs += start[n];
+          err = e.launch(one, blocks, b.stream);
+        } else if (!cb.add(n, start[n], per_n[n])) {
+          err = hipErrorInvalidValue;
+        }
+      }
+      if (cb.tasks && err == hipSuccess) err = cb.launch(s->variant, a, b.stream);
     }
     if (err == hipSuccess) {
       hipLaunchKernelGGL(serve_sum_kernel, dim3(nr), dim3(64), 0, b.stream, b.d_desc, b.d_mant,
@@ -410,6 +425,8 @@ int32_t lufqhe_server_create(int32_t walkers, const int32_t* h_walker_n, int32_t
     }
   }
   hipError_t err = hipGetDevice(&s->device);
+  if (err == hipSuccess)
+    err = hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, s->device);
   const size_t zb = s->z0.size() * sizeof(double2);
   if (err == hipSuccess) err = hipMalloc(&s->d_walker_z, zb);
   if (err == hipSuccess) err = hipMalloc(&s->d_perm, perm.size());

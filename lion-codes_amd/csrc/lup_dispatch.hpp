@@ -5,8 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lup_class.hpp"
 #include "lup_kernel.hpp"
-#include "lup_persistent.hpp"
 
 namespace lufqhe {
 
@@ -54,14 +54,44 @@ extern KernelEntry g_kernels[kNumVariants][kMaxN + 1][kMaxShapes];
 int selected_shape(int variant, int n);
 void set_selected_shape(int variant, int n, int shape);
 
-// Persistent mixed-size kernels (lup_persistent.hpp), one per fused variant
-// (0: CROUT_REF, 1: ABS) and size class, filled by lup_persist_inst.hip.
-using PersistLaunch = hipError_t (*)(const PersistArgs&, int64_t blocks, hipStream_t stream);
-struct PersistEntry {
-  PersistLaunch launch;
-  const void* kernel;  // for occupancy queries
+// Class kernels (lup_class.hpp), one per fused variant (0: CROUT_REF, 1: ABS)
+// and size class, filled by lup_class_inst.hip.
+using ClassLaunch = hipError_t (*)(const ClassArgs&, int64_t blocks, hipStream_t stream);
+constexpr int kClassVariants = 2;
+extern ClassLaunch g_class[kClassVariants][kClasses];
+
+// Whether a launch of `blocks` one-wave workgroups fills the device's wave
+// slots at two waves per SIMD.  From there on a size's own kernel wins, below
+// it a launch shared with the other sizes of the class: with all of a batch
+// of one size the class kernels take 1-5% longer (n <= 32) to 10-20% longer
+// (n >= 33, where they spill more), but 32768 matrices of n = 10..40 in 31
+// launches on four streams took 298 us and in shared ones 238.
+constexpr bool fills_device(int64_t blocks, int cus) { return blocks >= (int64_t)cus * 8; }
+
+// One class launch being put together: the buckets of its class, added
+// largest n first.
+struct ClassBatch {
+  int cls = 0;
+  int64_t tasks = 0;
+  double cost = 0.0;
+  int stream = 0;
+  ClassArgs ca{};
+
+  // matrices first .. first+count-1 of the index tables have side n
+  bool add(int n, int64_t first, int64_t count) {
+    const int b = ca.nbuckets++;
+    ca.n[b] = n;
+    ca.task[b] = (int32_t)tasks;
+    ca.first[b] = first;
+    ca.count[b] = count;
+    tasks += (count + class_group(n) - 1) / class_group(n);
+    return tasks <= INT32_MAX;  // a grid's size
+  }
+  hipError_t launch(int variant, const BatchArgs& args, hipStream_t s) const {
+    ClassArgs a = ca;
+    a.args = args;
+    return g_class[variant][cls](a, tasks, s);
+  }
 };
-constexpr int kPersistVariants = 2;
-extern PersistEntry g_persist[kPersistVariants][kPersistClasses];
 
 }  // namespace lufqhe
