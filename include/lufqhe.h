@@ -91,7 +91,11 @@ int32_t lufqhe_det_batched(const void *d_A, int64_t batch, int32_t n,
  * arithmetic, n).  Replaces the reference's fixed sizing, RunInfo::RunInfo
  * (LU-fqhe/src/RunInfo.cpp:46-78) and the matrices-per-block command-line
  * option (LU-fqhe/src/FQHE.cpp:214-265).  Selection is process wide; change
- * it while no launch of that n is being issued.  min_waves may be NULL. */
+ * it while no launch of that n is being issued.  A shape set here runs
+ * batches of every size; with a table's or the default shape, uniform batches
+ * too small to give every SIMD a wave (n = 17..32) or every compute unit a
+ * matrix (n >= 49) run a kernel of lower latency (all give the same bits).
+ * min_waves may be NULL. */
 int32_t lufqhe_shape_count(int32_t n);
 int32_t lufqhe_shape_info(int32_t n, int32_t shape, int32_t *lanes,
                           int32_t *lane_cols, int32_t *min_waves);

@@ -11,17 +11,22 @@ namespace lufqhe {
 // Filled at load time by the lup_inst.hip and lup_class_inst.hip objects.
 KernelEntry g_kernels[kNumVariants][kMaxN + 1][kMaxShapes];
 ClassLaunch g_class[kClassVariants][kClasses];
+SmallLaunch g_small[kClassVariants][kMaxN + 1];
 
 namespace {
 thread_local hipError_t t_last_hip = hipSuccess;
 std::atomic<int> g_selected[kNumVariants][kMaxN + 1];  // zero-initialised: shape 0
 }
 
+constexpr int kPinned = 0x100;
 int selected_shape(int variant, int n) {
-  return g_selected[variant][n].load(std::memory_order_relaxed);
+  return g_selected[variant][n].load(std::memory_order_relaxed) & ~kPinned;
 }
-void set_selected_shape(int variant, int n, int shape) {
-  g_selected[variant][n].store(shape, std::memory_order_relaxed);
+void set_selected_shape(int variant, int n, int shape, bool pinned) {
+  g_selected[variant][n].store(shape | (pinned ? kPinned : 0), std::memory_order_relaxed);
+}
+bool shape_pinned(int variant, int n) {
+  return (g_selected[variant][n].load(std::memory_order_relaxed) & kPinned) != 0;
 }
 
 // The kernel a launch of (variant, n) uses: the selected shape if it is
@@ -34,6 +39,23 @@ const KernelEntry& entry_for(int variant, int n) {
 int32_t hip_fail(hipError_t e) {
   t_last_hip = e;
   return LUFQHE_ERROR_HIP;
+}
+
+extern thread_local bool t_loading_table;  // lufqhe_table.cpp
+
+// A uniform batch: the selected shape's kernel, or the small batch's.
+hipError_t launch_uniform(const KernelEntry& e, int variant, int n, const BatchArgs& args,
+                          int64_t blocks, hipStream_t stream) {
+  if (args.count <= kSmallMost && variant < kClassVariants && g_small[variant][n] &&
+      !shape_pinned(variant, n)) {
+    int dev = 0, cus = 0;
+    hipError_t err = hipGetDevice(&dev);
+    if (err == hipSuccess)
+      err = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (err != hipSuccess) return err;
+    if (small_batch(n, args.count, cus)) return g_small[variant][n](args, stream);
+  }
+  return e.launch(args, blocks, stream);
 }
 
 hipError_t launch_inplace_write(double2* A, int64_t count, int64_t stride, const double2* mant,
@@ -124,7 +146,7 @@ int32_t lufqhe_det_batched(const void* d_A, int64_t batch, int32_t n,
   args.piv_stride = n;
   args.out = DetOut{static_cast<double2*>(d_mant), d_exp, d_logabs, d_phase,
                     d_info, d_piv};
-  const hipError_t err = e.launch(args, blocks, stream);
+  const hipError_t err = launch_uniform(e, v, n, args, blocks, stream);
   return err == hipSuccess ? LUFQHE_SUCCESS : hip_fail(err);
 }
 
@@ -152,7 +174,7 @@ int32_t lufqhe_fqhe_det(const void* d_z, int64_t count, int32_t n, int64_t z_str
   args.piv_stride = n;
   args.src = SRC_FQHE;
   args.out = DetOut{static_cast<double2*>(d_mant), d_exp, d_logabs, d_phase, d_info, d_piv};
-  const hipError_t err = e.launch(args, blocks, stream);
+  const hipError_t err = launch_uniform(e, v, n, args, blocks, stream);
   return err == hipSuccess ? LUFQHE_SUCCESS : hip_fail(err);
 }
 
@@ -192,7 +214,7 @@ int32_t lufqhe_set_shape(int32_t policy, int32_t arith, int32_t n, int32_t shape
   if (v < 0) return LUFQHE_ERROR_UNSUPPORTED;
   if (n < 1 || n > kMaxN || shape < 0 || shape >= kMaxShapes) return LUFQHE_ERROR_INVALID_VALUE;
   if (!g_kernels[v][n][shape].launch) return LUFQHE_ERROR_NOT_BUILT;
-  set_selected_shape(v, n, shape);
+  set_selected_shape(v, n, shape, !t_loading_table);
   return LUFQHE_SUCCESS;
 }
 

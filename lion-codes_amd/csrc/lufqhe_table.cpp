@@ -17,7 +17,17 @@
 
 #include "../../include/lufqhe.h"
 
+namespace lufqhe {
+// set while a table is applied: its shapes are not pinned
+thread_local bool t_loading_table = false;
+}  // namespace lufqhe
+
 namespace {
+
+struct LoadingTable {
+  LoadingTable() { lufqhe::t_loading_table = true; }
+  ~LoadingTable() { lufqhe::t_loading_table = false; }
+};
 
 bool read_file(const std::string& path, std::string& out) {
   FILE* f = std::fopen(path.c_str(), "rb");
@@ -71,6 +81,7 @@ extern "C" int32_t lufqhe_load_shape_table(const char* path) {
   if (p == std::string::npos) return -1;
   p = text.find('[', p);
   if (p == std::string::npos) return -1;
+  const LoadingTable loading;
   int32_t applied = 0;
   int depth = 0;
   size_t start = 0;

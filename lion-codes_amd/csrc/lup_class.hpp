@@ -45,7 +45,7 @@ constexpr int class_group(int n) { return 64 / class_shape(n).lanes; }  // matri
 
 constexpr int class_task_lds(int n) {
   const ShapeLC s = class_shape(n);
-  return s.panel ? panel_lds(n) : (64 / s.lanes) * group_lds(n, s.lanes, s.lane_cols);
+  return s.panel ? panel_lds(n, 64 / s.lanes, 1) : (64 / s.lanes) * group_lds(n, s.lanes, s.lane_cols);
 }
 constexpr int class_lds(int lo, int hi) {
   int m = 0;
@@ -74,7 +74,7 @@ __device__ __forceinline__ void class_dispatch(int n, const BatchArgs& args, int
     // shared with the other sizes and held from the dispatch on
     asm volatile("" : "+v"(lane));
     if constexpr (s.panel)
-      panel_task<LO, 64 / s.lanes, POLICY>(args, task, lds, lane);
+      panel_task<LO, 64 / s.lanes, 1, POLICY>(args, task, lds, lane, 0);
     else
       det_task<LO, s.lanes, s.lane_cols, POLICY, ARITH_FUSED>(args, task, lds, lane);
   } else {

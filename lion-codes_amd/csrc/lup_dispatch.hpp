@@ -51,14 +51,33 @@ struct KernelEntry {
 extern KernelEntry g_kernels[kNumVariants][kMaxN + 1][kMaxShapes];
 
 // Shape chosen per (variant, n); 0 until the autotuner's table is applied.
+// A shape set by lufqhe_set_shape is pinned: it runs batches of every size.
 int selected_shape(int variant, int n);
-void set_selected_shape(int variant, int n, int shape);
+void set_selected_shape(int variant, int n, int shape, bool pinned);
+bool shape_pinned(int variant, int n);
 
 // Class kernels (lup_class.hpp), one per fused variant (0: CROUT_REF, 1: ABS)
 // and size class, filled by lup_class_inst.hip.
 using ClassLaunch = hipError_t (*)(const ClassArgs&, int64_t blocks, hipStream_t stream);
 constexpr int kClassVariants = 2;
 extern ClassLaunch g_class[kClassVariants][kClasses];
+
+// Uniform batches that leave SIMDs idle are bound by one matrix's latency.
+// They run the panel kernel with one matrix per wave (n = 17..32: the pivot
+// row by v_readlane instead of LDS, and half the row slots) or two waves per
+// matrix (n >= 49: the trailing columns split between them).  Measured, us a
+// launch, against the selected shape: n = 17 9.1 / 13.5, n = 24 11.3 / 20.7,
+// n = 32 15.1 / 18.3, n = 56 29.2 / 36.1, n = 64 34.9 / 42.2 at 48 matrices;
+// n = 32 17.2 / 19.5 at 1024 and 23.5 / 22.4 at 2048; n = 64 35.4 / 42.6 at 256 and
+// 48.7 / 44.1 at 512.  At n = 33..48 two waves gained at most 9% and lost at
+// 512 matrices.
+constexpr int small_waves(int n) { return n < 17 ? 0 : n <= 32 ? 1 : n <= 48 ? 0 : 2; }
+constexpr bool small_batch(int n, int64_t count, int cus) {
+  return count <= (n <= 32 ? 4 : 1) * (int64_t)cus;
+}
+constexpr int64_t kSmallMost = 4 * 256;  // no larger batch is small on this architecture
+using SmallLaunch = hipError_t (*)(const BatchArgs&, hipStream_t stream);
+extern SmallLaunch g_small[kClassVariants][kMaxN + 1];
 
 // Whether a launch of `blocks` one-wave workgroups fills the device's wave
 // slots at two waves per SIMD.  From there on a size's own kernel wins, below

@@ -31,7 +31,7 @@ template <int N, int SH>
 constexpr auto kernel_of() {
   constexpr ShapeLC sh = shape_of<N, SH>();
   if constexpr (sh.panel)
-    return &lup_panel_kernel<N, 64 / sh.lanes, kPolicy, sh.waves>;
+    return &lup_panel_kernel<N, 64 / sh.lanes, 1, kPolicy, sh.waves>;
   else
     return &lup_det_kernel<N, sh.lanes, sh.lane_cols, kPolicy, kArith, kWavesPerBlock, sh.waves>;
 }
@@ -57,9 +57,20 @@ void register_shape() {
   }
 }
 
+// The kernel of a small batch (small_batch in lup_dispatch.hpp).
+template <int N>
+hipError_t launch_small(const BatchArgs& args, hipStream_t stream) {
+  constexpr int H = small_waves(N);
+  hipLaunchKernelGGL((lup_panel_kernel<N, 1, H, kPolicy, 2>), dim3((unsigned)args.count),
+                     dim3(64 * H), 0, stream, args);
+  return hipGetLastError();
+}
+
 template <int N>
 void register_one() {
   if constexpr (N % LUFQHE_SHARDS == LUFQHE_SHARD) {
+    if constexpr (kArith == ARITH_FUSED && small_waves(N) > 0)
+      g_small[LUFQHE_VARIANT][N] = &launch_small<N>;
     register_shape<N, 0>();
     register_shape<N, 1>();
     register_shape<N, 2>();

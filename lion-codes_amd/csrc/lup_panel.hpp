@@ -52,9 +52,13 @@ constexpr int kPanelStride = 5;
 constexpr int panel_row_stride(int n) { return ((4 * ((n + 3) / 4) + 11) / 16) * 16 + 4; }
 constexpr int panel_area(int g) { return 64 / g * kPanelStride + (g > 1 ? 8 : 0); }
 constexpr int panel_pivot_area(int n) { return 4 * panel_row_stride(n) + 8; }
-constexpr int panel_lds(int n) {
-  const int g = panel_groups(n);
+// One wave's own areas, and a workgroup's of h waves per matrix: with two
+// also the raw panels they hand each other (two, in turn) and their row maxima.
+constexpr int panel_wave_lds(int n, int g) {
   return g * (panel_area(g) + panel_pivot_area(n)) + (g > 1 ? g * 6 : 0) + 16;
+}
+constexpr int panel_lds(int n, int g, int h) {
+  return h * panel_wave_lds(n, g) + (h > 1 ? 2 * panel_area(1) + 64 : 0);
 }
 
 // Row slots a matrix still needs when panel p is searched (p = 0: all).  Once
@@ -67,8 +71,8 @@ constexpr int panel_lds(int n) {
 // 18.5 / 19.7, n = 52 24.1 / 30.8 (one slot less after the first panel, and so
 // no spills at two waves per SIMD), n = 64 48.7 / 50.4.
 constexpr int kMinPanelsLeft = 2;
-constexpr int panel_slots(int n, int p) {
-  const int rg = 16 / panel_groups(n), c = (n + 3) / 4;
+constexpr int panel_slots(int n, int g, int p) {
+  const int rg = 16 / g, c = (n + 3) / 4;
   int r = (n + rg - 1) / rg;
   for (int q = 0; q < p; ++q)
     if (r > 1 && n - 4 * (q + 1) <= (r - 1) * rg && c - 1 - q >= kMinPanelsLeft) --r;
@@ -78,20 +82,22 @@ constexpr int panel_slots(int n, int p) {
 struct PanelSlots {
   int at[17];
 };
-constexpr PanelSlots panel_slot_table(int n) {
+constexpr PanelSlots panel_slot_table(int n, int g) {
   PanelSlots t{};
-  for (int p = 0; p <= 16; ++p) t.at[p] = panel_slots(n, p);
+  for (int p = 0; p <= 16; ++p) t.at[p] = panel_slots(n, g, p);
   return t;
 }
 
-template <int N, int G>
+template <int N, int G, int H>
 struct PanelTile {
-  static constexpr PanelSlots slots = panel_slot_table(N);
+  static constexpr PanelSlots slots = panel_slot_table(N, G);
+  static_assert(H == 1 || (H == 2 && G == 1), "waves per matrix");
   static_assert(G == 1 || G == 2, "matrices per wave");
   static constexpr int L = 64 / G;             // panel layout: lanes (rows) per matrix
   static constexpr int RG = 16 / G;            // tile layout: lane-rows per matrix
   static constexpr int R = (N + RG - 1) / RG;  // row slots
   static constexpr int C = (N + 3) / 4;        // column slots = panels
+  static constexpr int CL = (C + H - 1) / H;   // column slots of one wave
   static_assert(N <= L && R * RG <= L, "one lane per row");
   static_assert(panel_row_stride(N) >= 4 * C, "a pivot row");
 };
@@ -230,13 +236,15 @@ __device__ __forceinline__ int select_group(const int (&v)[G], int g) {
   return r;
 }
 
-template <int N, int G, int POLICY>
+template <int N, int G, int H, int POLICY>
 __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
-                                           double2* __restrict__ lds, int lane) {
-  using T = PanelTile<N, G>;
-  constexpr int L = T::L, RG = T::RG, R = T::R, C = T::C;
+                                           double2* __restrict__ lds_all, int lane, int wave) {
+  using T = PanelTile<N, G, H>;
+  constexpr int L = T::L, RG = T::RG, R = T::R, C = T::C, CL = T::CL;
   constexpr int PS = kPanelStride, PG = panel_area(G);
   constexpr int US = panel_row_stride(N), GS = panel_pivot_area(N);
+  double2* lds = lds_all + (H > 1 ? wave * panel_wave_lds(N, G) : 0);
+  double2* shared = lds_all + H * panel_wave_lds(N, G);  // H > 1
   double2* pan = lds;               // the panel, then its multipliers
   double2* ub = pan + G * PG;       // its pivot rows
   double2* pv = ub + G * GS;        // G > 1: the pivot row of a step
@@ -251,13 +259,23 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
   // panel layout: one row (or column) per lane
   const int gp = lane / L, row = lane % L;
   double2* mine = pan + gp * PG + row * PS;           // this row of the panel
-  double2* tile = pan + gt * PG + rb * PS + jc;       // this lane's element of row slot 0
+  // this lane's element of row slot 0 and this row in raw panel p
+  auto raw_tile = [&](int p) {
+    return (H > 1 ? shared + (p & 1) * PG : pan + gt * PG) + rb * PS + jc;
+  };
+  auto raw_row = [&](int p) { return H > 1 ? shared + (p & 1) * PG + row * PS : mine; };
+  auto raw_sync = [&]() {
+    if constexpr (H > 1)
+      __syncthreads();
+    else
+      wave_lds_sync();
+  };
 
   const int64_t i_t = task * G + gt;
   const int64_t i_p = task * G + gp;
   const bool ok_t = i_t < args.count, ok_p = i_p < args.count;
 
-  double ax[R][C], ay[R][C];
+  double ax[R][CL], ay[R][CL];  // slot q holds columns 4 * (q * H + wave) ..
   int bad_perm = 0;
   if (args.src == SRC_FQHE) {
     double2 z = make_double2(0.0, 0.0);
@@ -290,9 +308,10 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
       wave_lds_sync();
 #pragma unroll
       for (int t = 0; t < R; ++t) {
-        const double2 v = tile[RG * t * PS];
-        ax[t][s] = v.x;
-        ay[t][s] = v.y;
+        if (H > 1 && s % H != wave) continue;
+        const double2 v = pan[gt * PG + (rb + RG * t) * PS + jc];
+        ax[t][s / H] = v.x;
+        ay[t][s / H] = v.y;
       }
       wave_lds_sync();
     }
@@ -311,15 +330,15 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
         if (perm) src = min((int)perm[r], N - 1);
         const double2* __restrict__ rp = base + (int64_t)src * ld;
 #pragma unroll
-        for (int s = 0; s < C; ++s) {
-          const int col = jc + 4 * s;
+        for (int q = 0; q < CL; ++q) {
+          const int col = jc + 4 * (q * H + wave);
           const double2 v = (col < N) ? rp[col] : make_double2(0.0, 0.0);
-          ax[t][s] = v.x;
-          ay[t][s] = v.y;
+          ax[t][q] = v.x;
+          ay[t][q] = v.y;
         }
       } else {
 #pragma unroll
-        for (int s = 0; s < C; ++s) ax[t][s] = ay[t][s] = 0.0;
+        for (int q = 0; q < CL; ++q) ax[t][q] = ay[t][q] = 0.0;
       }
     }
     if (args.row_perm && ok_p && row < N) {
@@ -335,18 +354,19 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
   int rej = -1;
   int want = G;
   if constexpr (POLICY == POLICY_CROUT_REF) {
-    double* scd = reinterpret_cast<double*>(pan);
+    double* scd = reinterpret_cast<double*>(H > 1 ? shared + 2 * PG : pan);
 #pragma unroll
     for (int t = 0; t < R; ++t) {
       double m = fabs(ax[t][0]);
 #pragma unroll
-      for (int s = 1; s < C; ++s)
-        if (jc + 4 * s < N) m = vmax_f64(m, fabs(ax[t][s]));
+      for (int q = 1; q < CL; ++q)
+        if (jc + 4 * (q * H + wave) < N) m = vmax_f64(m, fabs(ax[t][q]));
       m = lanerow_max<4>(m);
-      if (jc == 0) scd[gt * L + rb + RG * t] = m;
+      if (jc == 0) scd[wave * 64 + gt * L + rb + RG * t] = m;
     }
-    wave_lds_sync();
-    const double m = scd[lane];
+    raw_sync();
+    double m = scd[lane];
+    if constexpr (H > 1) m = vmax_f64(m, scd[64 + lane]);
     wave_lds_sync();
     const bool bad = row < N && m < kRowScaleMin;
     sc = (row < N && !bad) ? m : 1.0;
@@ -366,14 +386,16 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
   const double* pd = reinterpret_cast<const double*>(pan);
   const double* ud = reinterpret_cast<const double*>(ub);
   const unsigned odd = (ti & 1) ? 0x80000000u : 0u;  // operand lanes with k odd
-  const int ubase = (gt * GS + (ti >> 1) * US + jc) * 2 + (ti & 1);
-  const int ubase_y = (gt * GS + (ti >> 1) * US + jc) * 2 + ((ti & 1) ^ 1);
+  const int ubase = (gt * GS + (ti >> 1) * US + 4 * wave + jc) * 2 + (ti & 1);
+  const int ubase_y = (gt * GS + (ti >> 1) * US + 4 * wave + jc) * 2 + ((ti & 1) ^ 1);
 
   // panel 0 to LDS
+  if (H == 1 || wave == 0) {
+    double2* tile = raw_tile(0);
 #pragma unroll
-  for (int t = 0; t < R; ++t)
-    tile[RG * t * PS] = make_double2(ax[t][0], ay[t][0]);
-  wave_lds_sync();
+    for (int t = 0; t < R; ++t) tile[RG * t * PS] = make_double2(ax[t][0], ay[t][0]);
+  }
+  raw_sync();
 
 #pragma unroll
   for (int p = 0; p < C; ++p) {
@@ -381,6 +403,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
     const int nb = N - 4 * p < W ? N - 4 * p : W;
     const int R1 = T::slots.at[p], R2 = T::slots.at[p + 1];
     const bool trail = p + 1 < C;
+    const int q0 = (p + 1) / H;  // the first of a wave's slots that may lie beyond the panel
     double px[W], py[W];
     int pa[W];  // LDS row of each pivot (double2)
     int pj = -1, tj[R];
@@ -389,7 +412,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
 #pragma unroll
     for (int c = 0; c < W; ++c) {
       if (c >= nb) continue;
-      const double2 v = mine[c];
+      const double2 v = raw_row(p)[c];
       px[c] = v.x;
       py[c] = v.y;
     }
@@ -470,10 +493,10 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
           if (t >= R1) continue;
           const int q = rb + RG * t == pt ? j : tj[t];
           if (q >= 0) {
-            double2* dst = ub + gt * GS + q * US + jc;
+            double2* dst = ub + gt * GS + q * US + 4 * wave + jc;
 #pragma unroll
-            for (int s = 0; s < C; ++s)
-              if (s > p) dst[4 * s] = make_double2(ax[t][s], ay[t][s]);
+            for (int c = 0; c < CL; ++c)
+              if (c >= q0) dst[4 * H * c] = make_double2(ax[t][c], ay[t][c]);
           }
         }
         wave_lds_sync();
@@ -595,11 +618,11 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
       static_assert(RG * (4 * SW + 1) <= L * PS, "staging area");
       double2* stage = pan + gt * PG;
 #pragma unroll
-      for (int s0 = 0; s0 < C; s0 += SW) {
-        if (s0 + SW <= p + 1) continue;
+      for (int s0 = 0; s0 < CL; s0 += SW) {
+        if (s0 + SW <= q0) continue;
 #pragma unroll
         for (int c = 0; c < SW; ++c)
-          if (s0 + c > p && s0 + c < C)
+          if (s0 + c >= q0 && s0 + c < CL)
             stage[rb * (4 * SW + 1) + 4 * c + jc] =
                 make_double2(ax[R1 - 1][s0 + c], ay[R1 - 1][s0 + c]);
         wave_lds_sync();
@@ -610,16 +633,16 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
           double2 v[SW];
 #pragma unroll
           for (int c = 0; c < SW; ++c)
-            if (s0 + c > p && s0 + c < C) v[c] = make_double2(ax[t][s0 + c], ay[t][s0 + c]);
+            if (s0 + c >= q0 && s0 + c < CL) v[c] = make_double2(ax[t][s0 + c], ay[t][s0 + c]);
           if (st[t] >= R2 * RG) {
             const double2* row_t = stage + (st[t] - R2 * RG) * (4 * SW + 1) + jc;
 #pragma unroll
             for (int c = 0; c < SW; ++c)
-              if (s0 + c > p && s0 + c < C) v[c] = row_t[4 * c];
+              if (s0 + c >= q0 && s0 + c < CL) v[c] = row_t[4 * c];
           }
 #pragma unroll
           for (int c = 0; c < SW; ++c)
-            if (s0 + c > p && s0 + c < C) {
+            if (s0 + c >= q0 && s0 + c < CL) {
               ax[t][s0 + c] = v[c].x;
               ay[t][s0 + c] = v[c].y;
             }
@@ -629,29 +652,35 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
     }
     // trailing update, the next panel first
 #pragma unroll
-    for (int s = 0; s < C; ++s) {
-      if (s <= p) continue;
-      double Bx[2], By[2];
+    for (int q = 0; q < CL; ++q) {
+      if (q < q0) continue;
+      if (H == 1 || q > q0 || q * H + wave > p) {
+        double Bx[2], By[2];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        Bx[h] = ud[ubase + (2 * h * US + 4 * s) * 2];
-        By[h] = neg_if(ud[ubase_y + (2 * h * US + 4 * s) * 2], odd);
-      }
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int t = 0; t < R; ++t) {
-          if (t >= R2) continue;
-          ax[t][s] = mfma_4x4x4(Ax[t][h], Bx[h], ax[t][s]);
-          ay[t][s] = mfma_4x4x4(Ax[t][h], By[h], ay[t][s]);
+        for (int h = 0; h < 2; ++h) {
+          Bx[h] = ud[ubase + (2 * h * US + 4 * H * q) * 2];
+          By[h] = neg_if(ud[ubase_y + (2 * h * US + 4 * H * q) * 2], odd);
         }
-      if (s == p + 1) {
 #pragma unroll
-        for (int t = 0; t < R; ++t)
-          if (t < R2) tile[RG * t * PS] = make_double2(ax[t][s], ay[t][s]);
-        wave_lds_sync();
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int t = 0; t < R; ++t) {
+            if (t >= R2) continue;
+            ax[t][q] = mfma_4x4x4(Ax[t][h], Bx[h], ax[t][q]);
+            ay[t][q] = mfma_4x4x4(Ax[t][h], By[h], ay[t][q]);
+          }
+      }
+      if (q == q0) {
+        if (H == 1 || (p + 1) % H == wave) {
+          double2* tile = raw_tile(p + 1);
+#pragma unroll
+          for (int t = 0; t < R; ++t)
+            if (t < R2) tile[RG * t * PS] = make_double2(ax[t][q], ay[t][q]);
+        }
+        if (H == 1) wave_lds_sync();
       }
     }
+    if (H > 1) raw_sync();
   }
 
   // sign of the row permutation: one per step whose pivot was not in place
@@ -669,7 +698,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
   res.e = de;
   res.info = (rej >= 0) ? -(rej + 1) : zfirst == 255 ? 0 : zfirst;
   if (args.row_perm && group_max_i<L>(bad_perm) > 0) res.info = kInfoBadPerm;
-  if (ok_p) {
+  if (ok_p && (H == 1 || wave == 0)) {
     const int64_t o = args.out_idx ? args.out_idx[i_p] : i_p;
     if (args.out.piv && row < N)
       args.out.piv[o * args.piv_stride + row] = (int8_t)(res.info < 0 ? -1 : prec);
@@ -677,12 +706,13 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
   }
 }
 
-template <int N, int G, int POLICY, int OCC>
-__global__ void __launch_bounds__(64, OCC) lup_panel_kernel(BatchArgs args) {
-  __shared__ double2 lds[panel_lds(N)];
+template <int N, int G, int H, int POLICY, int OCC>
+__global__ void __launch_bounds__(64 * H, OCC) lup_panel_kernel(BatchArgs args) {
+  __shared__ double2 lds[panel_lds(N, G, H)];
   const int64_t task = blockIdx.x;
-  if (task * G >= args.count) return;
-  panel_task<N, G, POLICY>(args, task, lds, (int)(threadIdx.x & 63));
+  if (task * G >= args.count) return;  // the whole workgroup
+  const int wave = H > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
+  panel_task<N, G, H, POLICY>(args, task, lds, (int)(threadIdx.x & 63), wave);
 }
 
 }  // namespace lufqhe

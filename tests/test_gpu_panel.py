@@ -82,3 +82,54 @@ def test_criteria_outside_the_corrected_range(lc, orc, wl, dev, n):
     A[7][:, 3] = 0.0
     A[7][n - 1, 3] = 2.0 ** -950
     check(lc, orc, dev, A)
+
+
+@pytest.mark.parametrize("n,limit", [(17, 1024), (20, 1024), (24, 1024), (25, 1024), (32, 1024),
+                                     (49, 256), (53, 256), (57, 256), (60, 256), (64, 256)])
+def test_small_batches(lc, orc, wl, dev, n, limit):
+    """The low-latency kernels of batches that leave SIMDs idle, on both sides
+    of the line where they end (256 compute units), in a padded layout."""
+    lc.apply_shape_table()  # a table's shapes are not pinned
+    base = wl.gaussian_np(64, n, seed=900 + n)
+    base[0] = np.round(base[0])
+    base[1] = np.round(base[1].real)
+    base[2, :, 3] = 0
+    base[3] *= 2.0 ** 980
+    for policy in ("crout_ref", "abs"):
+        o = orc.mirror(base, policy, "fused")
+        for count in (1, 2, 64, limit, limit + 1):
+            idx = np.arange(count) % 64
+            A = torch.zeros(count, n, n + 3, dtype=torch.complex128, device=dev)
+            A[:, :, :n] = torch.from_numpy(base[idx]).to(dev)
+            r = lc.det_batched(A[:, :, :n], policy=policy, pivots=True)
+            torch.cuda.synchronize()
+            what = (n, policy, count)
+            assert np.array_equal(r.info.cpu().numpy(), o["info"][idx]), what
+            assert same(r.mant.cpu().numpy(), o["mant"][idx]), what
+            assert np.array_equal(r.exp.cpu().numpy(), o["exp"][idx]), what
+            ok = o["info"][idx] >= 0
+            assert np.array_equal(r.piv.cpu().numpy()[ok].astype(np.int32), o["piv"][idx][ok]), what
+
+
+@pytest.mark.parametrize("n", [17, 24, 32, 49, 57, 64])
+def test_small_batches_built_on_the_device(lc, wl, dev, n):
+    """The same kernels building their matrices from permuted positions (one
+    permutation entry out of range) equal the pinned shape's."""
+    lc.apply_shape_table()
+    rng = np.random.default_rng(n)
+    z = torch.from_numpy(wl.fqhe_positions(n, rng)[None, :]).to(dev)
+    perm = np.argsort(rng.random((9, n)), axis=1).astype(np.uint8)
+    perm[4, n - 1] = n
+    p = torch.from_numpy(perm).to(dev)
+    small = lc.fqhe_det(z, row_perm=p, count=9, pivots=True)
+    sh = lc.get_shape("crout_ref", "fused", n)
+    try:
+        assert lc.set_shape("crout_ref", "fused", n, sh)  # pinned
+        big = lc.fqhe_det(z, row_perm=p, count=9, pivots=True)
+    finally:
+        lc.apply_shape_table()
+    torch.cuda.synchronize()
+    assert small.info.cpu().tolist() == big.info.cpu().tolist()
+    assert small.info[4].item() == -1000
+    assert torch.equal(small.piv, big.piv) and torch.equal(small.exp, big.exp)
+    assert same(small.mant.cpu().numpy(), big.mant.cpu().numpy())
