@@ -33,6 +33,8 @@
 #include <cmath>
 #include <cstring>
 #include <deque>
+#include <memory>
+#include <mutex>
 #include <new>
 #include <thread>
 #include <vector>
@@ -156,30 +158,6 @@ static_assert(sizeof(lufqhe_serve_stats) == 120, "lufqhe_serve_stats layout");
 static_assert(sizeof(lufqhe_serve_record) == 64, "lufqhe_serve_record layout");
 static_assert(sizeof(ReqDesc) == 64, "ReqDesc layout");
 
-}  // namespace
-
-// ---------------------------------------------------------------- server
-struct lufqhe_server {
-  int device = 0;
-  int cus = 0;  // compute units of the device
-  int variant = 0;
-  int walkers = 0;
-  int perms = 0;
-  uint64_t seed = 0;
-  std::vector<int32_t> wn;            // n per walker
-  std::vector<double2> z0;            // initial configurations [walkers][64]
-  double2* d_walker_z = nullptr;      // [walkers][64]
-  uint8_t* d_perm = nullptr;          // [walkers][perms][64]
-  int64_t resident_bytes = 0;
-
-  ~lufqhe_server() {
-    if (d_walker_z) (void)hipFree(d_walker_z);
-    if (d_perm) (void)hipFree(d_perm);
-  }
-};
-
-namespace {
-
 // Per-request record of a run.
 struct Req {
   int64_t id;
@@ -212,39 +190,15 @@ struct BatchSlot {
   int64_t bytes = 0;
 };
 
-// Device bytes a request holds while in flight: per term its tables (24 B)
-// and outputs (mant + exp, 20 B); its descriptor, sum and configuration slot.
-inline int64_t request_bytes(int k) {
-  return (int64_t)k * (24 + 20) + (int64_t)sizeof(ReqDesc) + 20 + kSlotZ * 16;
-}
-
-// Batch buffers of one in-flight slot and the configuration slots: device
-// bytes a run allocates up front.
-int64_t slot_bytes(int64_t R, int64_t D) {
-  return align256(R * (int64_t)sizeof(ReqDesc)) + 3 * align256(D * 8) + align256(D * 16) +
-         align256(D * 4) + align256(R * 16) + align256(R * 4);
-}
-int64_t arena_bytes(const lufqhe_serve_config& c, int walkers) {
-  const int64_t slots = (int64_t)c.max_inflight * c.max_batch_requests + walkers;
-  return c.max_inflight * slot_bytes(c.max_batch_requests, c.max_batch_dets) +
-         slots * kSlotZ * (int64_t)sizeof(double2);
-}
-
-struct Run {
-  lufqhe_server* s;
-  lufqhe_serve_config cfg;
-  int64_t arena_bytes = 0;
+// What a run allocates: its batch slots and the configuration slots.
+struct RunBuffers {
+  int inflight = 0;
+  int64_t R = 0, D = 0;  // requests and determinants of a batch
   std::vector<BatchSlot> bs;
   double2* d_slot_z = nullptr;
-  std::vector<int32_t> free_slots;
-  // walker state
-  std::vector<int32_t> commit;   // slot with the accepted, uncommitted configuration
-  std::vector<double> log_psi;   // log|psi| of the accepted configuration
-  std::vector<char> busy;
-  std::vector<std::deque<int64_t>> queue;  // arrived requests per walker
-  std::deque<int> ready;                   // walkers with a queued request, FIFO by arrival
+  int64_t nslots = 0;
 
-  ~Run() {
+  ~RunBuffers() {
     for (auto& b : bs) {
       if (b.done) (void)hipEventDestroy(b.done);
       if (b.stream) (void)hipStreamDestroy(b.stream);
@@ -256,10 +210,15 @@ struct Run {
     if (d_slot_z) (void)hipFree(d_slot_z);
   }
 
-  hipError_t alloc() {
-    const int nb = cfg.max_inflight;
-    const int64_t R = cfg.max_batch_requests, D = cfg.max_batch_dets;
-    bs.resize(nb);
+  bool fits(const lufqhe_serve_config& c) const {
+    return inflight == c.max_inflight && R == c.max_batch_requests && D == c.max_batch_dets;
+  }
+
+  hipError_t alloc(const lufqhe_serve_config& c, int walkers) {
+    inflight = c.max_inflight;
+    R = c.max_batch_requests;
+    D = c.max_batch_dets;
+    bs.resize(inflight);
     hipError_t err = hipSuccess;
     for (auto& b : bs) {
       if (err == hipSuccess) err = hipStreamCreateWithFlags(&b.stream, hipStreamNonBlocking);
@@ -290,12 +249,72 @@ struct Run {
       b.d_sum_e = reinterpret_cast<int32_t*>(base + o_se);
     }
     // configuration slots: every request in flight plus one held per walker
-    const int64_t nslots = (int64_t)nb * R + s->walkers;
+    nslots = (int64_t)inflight * R + walkers;
     if (err == hipSuccess) err = hipMalloc(&d_slot_z, nslots * kSlotZ * sizeof(double2));
-    free_slots.clear();
-    for (int64_t i = nslots - 1; i >= 0; --i) free_slots.push_back((int32_t)i);
     return err;
   }
+};
+
+}  // namespace
+
+// ---------------------------------------------------------------- server
+struct lufqhe_server {
+  int device = 0;
+  int cus = 0;  // compute units of the device
+  int variant = 0;
+  int walkers = 0;
+  int perms = 0;
+  uint64_t seed = 0;
+  std::vector<int32_t> wn;            // n per walker
+  std::vector<double2> z0;            // initial configurations [walkers][64]
+  double2* d_walker_z = nullptr;      // [walkers][64]
+  uint8_t* d_perm = nullptr;          // [walkers][perms][64]
+  int64_t resident_bytes = 0;
+  // The buffers of the last run, for one with the same limits: allocating and
+  // freeing them (pinned memory, streams, device blocks) took 2 of the 5 ms of
+  // a 384-request run.  At most one set, freed with the server or by a run with
+  // other limits; runs that overlap allocate their own.
+  std::mutex mu;
+  std::unique_ptr<RunBuffers> kept;
+
+  ~lufqhe_server() {
+    if (d_walker_z) (void)hipFree(d_walker_z);
+    if (d_perm) (void)hipFree(d_perm);
+  }
+};
+
+namespace {
+
+// Device bytes a request holds while in flight: per term its tables (24 B)
+// and outputs (mant + exp, 20 B); its descriptor, sum and configuration slot.
+inline int64_t request_bytes(int k) {
+  return (int64_t)k * (24 + 20) + (int64_t)sizeof(ReqDesc) + 20 + kSlotZ * 16;
+}
+
+// Batch buffers of one in-flight slot and the configuration slots: device
+// bytes a run allocates up front.
+int64_t slot_bytes(int64_t R, int64_t D) {
+  return align256(R * (int64_t)sizeof(ReqDesc)) + 3 * align256(D * 8) + align256(D * 16) +
+         align256(D * 4) + align256(R * 16) + align256(R * 4);
+}
+int64_t arena_bytes(const lufqhe_serve_config& c, int walkers) {
+  const int64_t slots = (int64_t)c.max_inflight * c.max_batch_requests + walkers;
+  return c.max_inflight * slot_bytes(c.max_batch_requests, c.max_batch_dets) +
+         slots * kSlotZ * (int64_t)sizeof(double2);
+}
+
+struct Run {
+  lufqhe_server* s;
+  lufqhe_serve_config cfg;
+  int64_t arena_bytes = 0;
+  std::unique_ptr<RunBuffers> buf;
+  std::vector<int32_t> free_slots;
+  // walker state
+  std::vector<int32_t> commit;   // slot with the accepted, uncommitted configuration
+  std::vector<double> log_psi;   // log|psi| of the accepted configuration
+  std::vector<char> busy;
+  std::vector<std::deque<int64_t>> queue;  // arrived requests per walker
+  std::deque<int> ready;                   // walkers with a queued request, FIFO by arrival
 
   // Launch batch `b` holding b.reqs.
   hipError_t launch(BatchSlot& b) {
@@ -332,12 +351,12 @@ struct Run {
                                     hipMemcpyHostToDevice, b.stream);
     if (err == hipSuccess) {
       hipLaunchKernelGGL(serve_prepare_kernel, dim3(nr), dim3(256), 0, b.stream, b.d_desc,
-                         s->d_walker_z, d_slot_z, s->perms, b.d_offs, b.d_perm_offs,
+                         s->d_walker_z, buf->d_slot_z, s->perms, b.d_offs, b.d_perm_offs,
                          b.d_out_idx);
       err = hipGetLastError();
     }
     BatchArgs a{};
-    a.A = d_slot_z;
+    a.A = buf->d_slot_z;
     a.offs = b.d_offs;
     a.out_idx = b.d_out_idx;
     a.row_perm = s->d_perm;
@@ -489,8 +508,18 @@ int32_t lufqhe_server_run(lufqhe_server* s, const lufqhe_serve_config* cfg,
   run.s = s;
   run.cfg = *cfg;
   run.arena_bytes = arena;
-  err = run.alloc();
-  if (err != hipSuccess) return hip_fail(err);
+  {
+    std::lock_guard<std::mutex> lock(s->mu);
+    if (s->kept && s->kept->fits(*cfg)) run.buf = std::move(s->kept);
+    s->kept.reset();
+  }
+  if (!run.buf) {
+    run.buf.reset(new (std::nothrow) RunBuffers());
+    if (!run.buf) return LUFQHE_ERROR_HIP;
+    err = run.buf->alloc(*cfg, s->walkers);
+    if (err != hipSuccess) return hip_fail(err);
+  }
+  for (int64_t i = run.buf->nslots - 1; i >= 0; --i) run.free_slots.push_back((int32_t)i);
   const int W = s->walkers;
   run.commit.assign(W, -1);
   run.log_psi.assign(W, -INFINITY);
@@ -539,7 +568,7 @@ int32_t lufqhe_server_run(lufqhe_server* s, const lufqhe_serve_config* cfg,
       progressed = true;
     }
     // 2. completions
-    for (auto& b : run.bs) {
+    for (auto& b : run.buf->bs) {
       if (!b.busy) continue;
       const hipError_t q = hipEventQuery(b.done);
       if (q == hipErrorNotReady) continue;
@@ -591,7 +620,7 @@ int32_t lufqhe_server_run(lufqhe_server* s, const lufqhe_serve_config* cfg,
     }
     if (err != hipSuccess) break;
     // 3. admission and launch: fill a free batch slot from the ready walkers
-    for (auto& b : run.bs) {
+    for (auto& b : run.buf->bs) {
       if (b.busy || run.ready.empty()) continue;
       int64_t bdets = 0, bbytes = 0;
       while (!run.ready.empty() && (int64_t)b.reqs.size() < cfg->max_batch_requests) {
@@ -632,7 +661,7 @@ int32_t lufqhe_server_run(lufqhe_server* s, const lufqhe_serve_config* cfg,
     }
   }
   if (err != hipSuccess) {
-    for (auto& b : run.bs)
+    for (auto& b : run.buf->bs)
       if (b.stream) (void)hipStreamSynchronize(b.stream);
     return hip_fail(err);
   }
@@ -652,13 +681,13 @@ int32_t lufqhe_server_run(lufqhe_server* s, const lufqhe_serve_config* cfg,
       fin.push_back(d);
     }
     if (!fin.empty()) {
-      BatchSlot& b = run.bs[0];
+      BatchSlot& b = run.buf->bs[0];
       for (size_t i = 0; i < fin.size(); i += cfg->max_batch_requests) {
         const int nr = (int)std::min<size_t>(cfg->max_batch_requests, fin.size() - i);
         err = hipMemcpy(b.d_desc, fin.data() + i, nr * sizeof(ReqDesc), hipMemcpyHostToDevice);
         if (err != hipSuccess) break;
         hipLaunchKernelGGL(serve_prepare_kernel, dim3(nr), dim3(256), 0, b.stream, b.d_desc,
-                           s->d_walker_z, run.d_slot_z, s->perms, b.d_offs, b.d_perm_offs,
+                           s->d_walker_z, run.buf->d_slot_z, s->perms, b.d_offs, b.d_perm_offs,
                            b.d_out_idx);
         err = hipGetLastError();
         if (err == hipSuccess) err = hipStreamSynchronize(b.stream);
@@ -667,6 +696,11 @@ int32_t lufqhe_server_run(lufqhe_server* s, const lufqhe_serve_config* cfg,
     }
   }
   if (err != hipSuccess) return hip_fail(err);
+  {
+    // every batch has completed and the last commit was waited for
+    std::lock_guard<std::mutex> lock(s->mu);
+    if (!s->kept) s->kept = std::move(run.buf);
+  }
 
   if (stats) {
     std::vector<double> lat(latency);
