@@ -5,10 +5,11 @@
 //
 //   tile layout   The whole matrix stays in registers in the result layout of
 //                 v_mfma_f64_4x4x4_4b: lane = col + 4*block + 16*i.  A wave
-//                 holds G = 2 matrices (n <= 32) or one; a matrix has 16/G
-//                 lane-rows by 4 lane-columns, R row slots and C column slots,
-//                 and the real and imaginary parts are separate registers.
-//                 Column slot p is panel p.
+//                 holds G = 2 matrices (n <= 32, in batches that fill the
+//                 device) or one; a matrix has 16/G lane-rows by 4
+//                 lane-columns, R row slots and C column slots, and the real
+//                 and imaginary parts are separate registers.  Column slot p
+//                 is panel p.
 //   panel layout  A panel (four columns of every row) goes through LDS into
 //                 one row per lane.  Its four steps -- pivot search, pivot row
 //                 to every lane, reciprocal, multipliers, update of the
@@ -31,11 +32,18 @@
 //
 // What bounds it.  MFMA and vector instructions share one FP64 pipe (they do
 // not overlap, and alternating them is slower than running them in runs), so
-// a step costs its issue: n = 32 runs about 58 vector instructions and 14
-// MFMAs of 16 cycles per step for two matrices, where lup_det_kernel's step
-// took 190 instructions; the rest is the latency of the serial search,
-// broadcast and reciprocal, which two waves per SIMD cover to about two
-// thirds.
+// a step costs its issue: an n = 32 wave (two matrices) issues 3814
+// instructions, 312 of them MFMAs of 16 cycles, where lup_det_kernel issued
+// 6167; at two waves per SIMD they fill 72% of the cycles and LDS is busy for
+// 51%.  The rest is the latency of the serial search, pivot row and
+// reciprocal.  65536 x n = 32: 475 -> 396 us; above n = 56 the tile leaves
+// room for one wave per SIMD only (n = 64: 82 -> 49 ns per determinant).
+//
+// H = 2 (one matrix, two waves) is for batches with fewer matrices than CUs,
+// where a wave has a SIMD to itself and the trailing update is most of its
+// time: both waves take the panel's steps, each holds and updates every other
+// column slot, and a raw panel goes to the other wave through one of two
+// shared buffers, with one barrier per panel.
 #pragma once
 
 #include "lup_kernel.hpp"
@@ -55,7 +63,7 @@ constexpr int panel_pivot_area(int n) { return 4 * panel_row_stride(n) + 8; }
 // One wave's own areas, and a workgroup's of h waves per matrix: with two
 // also the raw panels they hand each other (two, in turn) and their row maxima.
 constexpr int panel_wave_lds(int n, int g) {
-  return g * (panel_area(g) + panel_pivot_area(n)) + (g > 1 ? g * 6 : 0) + 16;
+  return g * (panel_area(g) + panel_pivot_area(n)) + 16;
 }
 constexpr int panel_lds(int n, int g, int h) {
   return h * panel_wave_lds(n, g) + (h > 1 ? 2 * panel_area(1) + 64 : 0);
@@ -67,9 +75,11 @@ constexpr int panel_lds(int n, int g, int h) {
 // their trailing columns through the panel's LDS area (one slot is written,
 // only the places that take a row read), the row's state by ds_bpermute.  All
 // later panels then update, write and read one slot less.  Measured with and
-// without, ns per determinant: n = 32 6.55 / 6.88, n = 40 13.4 / 14.6, n = 48
-// 18.5 / 19.7, n = 52 24.1 / 30.8 (one slot less after the first panel, and so
-// no spills at two waves per SIMD), n = 64 48.7 / 50.4.
+// without, ns per determinant: n = 32 6.55 / 6.88 (with pivot rows still passed
+// through LDS; now 6.33), n = 40 13.4 / 14.6, n = 48 18.5 / 19.7, n = 52
+// 24.1 / 30.8 (one slot less after the first panel, and so no spills at two
+// waves per SIMD), n = 64 48.7 / 50.4.  kMinPanelsLeft = 1, 3 and 4 are within
+// 1% at n = 26..64.
 constexpr int kMinPanelsLeft = 2;
 constexpr int panel_slots(int n, int g, int p) {
   const int rg = 16 / g, c = (n + 3) / 4;
@@ -247,8 +257,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
   double2* shared = lds_all + H * panel_wave_lds(N, G);  // H > 1
   double2* pan = lds;               // the panel, then its multipliers
   double2* ub = pan + G * PG;       // its pivot rows
-  double2* pv = ub + G * GS;        // G > 1: the pivot row of a step
-  int* pjv = reinterpret_cast<int*>(pv + (G > 1 ? G * 6 : 0));  // step each row was pivot of
+  int* pjv = reinterpret_cast<int*>(ub + G * GS);  // step each row was pivot of
 
   // tile layout (MFMA 4x4x4 result): lane = col + 4*block + 16*i
   const int jc = lane & 3, blk = (lane >> 2) & 3, ti = lane >> 4;
@@ -409,6 +418,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
     int pj = -1, tj[R];
     double Ax[R][2];
     double2 uc[W];
+    double2 u[W][W], lp[W][W];  // G > 1: pivot rows after their steps, their multipliers
 #pragma unroll
     for (int c = 0; c < W; ++c) {
       if (c >= nb) continue;
@@ -440,27 +450,49 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
               uy[cc] = readlane_d(py[cc], pl);
             }
         } else {
-          // the other lanes write to the part of their panel row that is free
-          double2* w = __builtin_amdgcn_inverse_ballot_w64(m) ? pv + gp * 6 : mine + j;
-          w[0] = make_double2(px[j], py[j]);
-          *reinterpret_cast<int2*>(w + nb - j) = make_int2(pos, gp * PG + row * PS);
-#pragma unroll
-          for (int cc = 0; cc < W; ++cc)
-            if (cc > j && cc < nb) w[cc - j] = make_double2(px[cc], py[cc]);
           wave_lds_sync();
-          const double2* r = pv + gp * 6;
-          const double2 v = r[0];
-          const int2 pi = *reinterpret_cast<const int2*>(r + nb - j);
-          ux[j] = v.x;
-          uy[j] = v.y;
-          ppos = pi.x;
-          pa[j] = pi.y;
+          // The row as the panel began it and its multipliers are in LDS: every
+          // lane reads those and takes the row's earlier steps itself (64 more
+          // instructions per panel, but no write that a read then waits for:
+          // LDS moves 64 B per clock and CU on writes and was busy for 70% of
+          // n = 32; 6.59 -> 6.33 ns per determinant there, 5.06 -> 4.90 at
+          // n = 26).  With one matrix per wave v_readlane is as fast (n = 40)
+          // or faster (n = 64, 4%).
+          int pl[G];
+#pragma unroll
+          for (int g = 0; g < G; ++g) pl[g] = group_first<G>(m, g);
+          int pp[G], at[G];
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            pp[g] = __builtin_amdgcn_readlane(pos, g * L + pl[g]);
+            at[g] = g * PG + pl[g] * PS;
+          }
+          ppos = select_group<G>(pp, gp);
+          pa[j] = select_group<G>(at, gp);
+          const double2* r = pan + pa[j];
+          double2 v[W];
 #pragma unroll
           for (int cc = 0; cc < W; ++cc)
-            if (cc > j && cc < nb) {
-              const double2 q = r[cc - j];
-              ux[cc] = q.x;
-              uy[cc] = q.y;
+            if (cc < nb) v[cc] = r[cc];
+#pragma unroll
+          for (int q = 0; q < W; ++q)
+            if (q < j) {
+              lp[j][q] = v[q];
+#pragma unroll
+              for (int cc = 0; cc < W; ++cc)
+                if (cc >= j && cc < nb) {
+                  v[cc].x = fma(v[q].x, u[q][cc].x, v[cc].x);
+                  v[cc].y = fma(v[q].x, u[q][cc].y, v[cc].y);
+                  v[cc].x = fma(v[q].y, u[q][cc].y, v[cc].x);
+                  v[cc].y = fma(-v[q].y, u[q][cc].x, v[cc].y);
+                }
+            }
+#pragma unroll
+          for (int cc = 0; cc < W; ++cc)
+            if (cc >= j && cc < nb) {
+              ux[cc] = v[cc].x;
+              uy[cc] = v[cc].y;
+              u[j][cc] = v[cc];
             }
           wave_lds_sync();
         }
@@ -509,7 +541,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
         for (int i = 1; i < W; ++i)
 #pragma unroll
           for (int q = 0; q < W; ++q)
-            if (q < i) l[i][q] = pan[pa[i] + q];
+            if (q < i) l[i][q] = G > 1 ? lp[i][q] : pan[pa[i] + q];
 #pragma unroll
         for (int q = 0; q < W; ++q)
 #pragma unroll
@@ -552,7 +584,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
         const double ly = fma(py[j], ir, px[j] * ii);
         double nl = -lx;
         asm("" : "+v"(nl));
-        if (trail) mine[j] = make_double2(nl, ly);
+        if (trail || (G > 1 && j + 1 < nb)) mine[j] = make_double2(nl, ly);
 #pragma unroll
         for (int cc = 0; cc < W; ++cc)
           if (cc > j && cc < nb) {
