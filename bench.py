@@ -44,14 +44,16 @@ OUT_BYTES = 16 + 4 + 8 + 8 + 4   # mant, exp, logabs, phase, info
 # (FETCH_SIZE and WRITE_SIZE, one counter per run, each scaled by what the
 # same counter reads for a plain 1 GiB device copy: x2.0 and x1.0;
 # profiles/lup_det_kernel_hbm_counters.md).
-MEASURED_TRAFFIC_N32 = 1.0799e9
+MEASURED_TRAFFIC_N32 = 1.0796e9
 # FP64 instructions one launch of the n=32 kernel issues, per wave (a wave
 # factors two matrices; 32768 waves per launch), measured with rocprofv3
-# (SQ_INSTS_VALU_FMA_F64, _MUL_F64, _ADD_F64 and SQ_INSTS_VALU;
-# profiles/lup_det_kernel_sizes_sq_counters.md).  Every one runs on all 64
-# lanes, so the FP64 flop the hardware executes per launch is
-# 32768 x 64 x (2 FMA + MUL + ADD).
-MEASURED_F64_N32 = {"waves": 32768, "fma": 2317.0, "mul": 318.0, "add": 48.0, "valu": 6167.0}
+# (SQ_INSTS_VALU_FMA_F64, _MUL_F64, _ADD_F64, SQ_INSTS_VALU_MFMA_F64 and
+# SQ_INSTS_VALU; profiles/lup_det_kernel_sizes_sq_counters.md).  Every one
+# runs on all 64 lanes and an MFMA (4x4x4, four blocks) is four FMAs per
+# lane, so the FP64 flop the hardware executes per launch is
+# 32768 x 64 x (2 FMA + MUL + ADD + 8 MFMA).
+MEASURED_F64_N32 = {"waves": 32768, "fma": 1127.0, "mul": 268.0, "add": 48.0, "mfma": 312.0,
+                    "valu": 3814.0}
 DEVICE_WARM_S = 0.25  # untimed device warm-up before the W warm-up steps
 
 
@@ -64,10 +66,10 @@ def fp64_counter(kern_ms: float) -> dict:
     launch (rocprofv3 instruction counts, all 64 lanes) over the live kernel
     time, and the FP64 instructions' share of the VALU instructions."""
     m = MEASURED_F64_N32
-    flop = m["waves"] * 64 * (2 * m["fma"] + m["mul"] + m["add"])
+    flop = m["waves"] * 64 * (2 * m["fma"] + m["mul"] + m["add"] + 8 * m["mfma"])
     tflops = flop / (kern_ms * 1e-3) / 1e12
     return {"executed_flop_per_launch": flop, "tflops": tflops, "frac": tflops / FP64_PEAK_TFLOPS,
-            "f64_share_of_valu": (m["fma"] + m["mul"] + m["add"]) / m["valu"],
+            "f64_share_of_valu": (m["fma"] + m["mul"] + m["add"] + m["mfma"]) / m["valu"],
             "source": "profiles/lup_det_kernel_sizes_sq_counters.md"}
 
 
@@ -269,8 +271,8 @@ def bench_small_batch(lc, wl, dev, reps: int, samples: dict) -> dict:
 
 def bench_mixed(lc, wl, dev, reps: int, samples: dict) -> dict:
     """Mixed-size batch: 200000 matrices, n ~ U{8..64}, 5% near-singular; one
-    hipGraph replay of the bucketed plan (per-size launches over streams, or
-    the persistent class kernels) vs per-size plain launches."""
+    hipGraph replay of the bucketed plan (per-size and class launches over
+    streams) vs per-size plain launches."""
     import torch
     count, seed = 200000, 2024
     flat, ns, offs, sing = wl.mixed_batch(count, seed, device=dev)
