@@ -91,18 +91,35 @@ int32_t lufqhe_det_batched(const void *d_A, int64_t batch, int32_t n,
  * arithmetic, n).  Replaces the reference's fixed sizing, RunInfo::RunInfo
  * (LU-fqhe/src/RunInfo.cpp:46-78) and the matrices-per-block command-line
  * option (LU-fqhe/src/FQHE.cpp:214-265).  Selection is process wide; change
- * it while no launch of that n is being issued.  A shape set here runs
- * batches of every size; with a table's or the default shape, uniform batches
- * too small to give every SIMD a wave (n = 17..32) or every compute unit a
- * matrix (n >= 49) run a kernel of lower latency (all give the same bits).
- * min_waves may be NULL. */
+ * it while no launch of that n is being issued.  min_waves may be NULL.
+ *
+ * Each (policy, arithmetic, n) has a default shape: 0, or what the last table
+ * or lufqhe_set_default_shape named.  While it is selected, uniform batches
+ * (lufqhe_det_batched, lufqhe_fqhe_det, lufqhe_det_inplace*) too small to give
+ * every SIMD a wave (n = 17..32) or every compute unit a matrix (n >= 49) run a
+ * kernel of lower latency.  Any other shape given to lufqhe_set_shape runs
+ * uniform batches of every size, and so does the default one given as shape |
+ * LUFQHE_SHAPE_PINNED.  lufqhe_get_shape returns what lufqhe_set_shape was
+ * given, flag included, so get, set, and set with the value got restores the
+ * selection.  Mixed plans and the server say below where they use it.  All
+ * kernels give the same bits. */
+#define LUFQHE_SHAPE_PINNED 0x100
+#define LUFQHE_SHAPE_SMALL_BATCH 0x200
 int32_t lufqhe_shape_count(int32_t n);
 int32_t lufqhe_shape_info(int32_t n, int32_t shape, int32_t *lanes,
                           int32_t *lane_cols, int32_t *min_waves);
 int32_t lufqhe_set_shape(int32_t policy, int32_t arith, int32_t n,
                          int32_t shape);
+/* Selects a shape and makes it the default, as a table's entry does. */
+int32_t lufqhe_set_default_shape(int32_t policy, int32_t arith, int32_t n,
+                                 int32_t shape);
 /* The selected shape, or -1 for invalid arguments. */
 int32_t lufqhe_get_shape(int32_t policy, int32_t arith, int32_t n);
+/* The shape a uniform batch of `batch` >= 1 matrices runs now, or
+ * LUFQHE_SHAPE_SMALL_BATCH for the kernel of small batches; compute_units 0
+ * asks the current device.  -1 for invalid arguments or if it cannot be asked. */
+int32_t lufqhe_uniform_shape(int32_t policy, int32_t arith, int32_t n,
+                             int64_t batch, int32_t compute_units);
 /* Applies a shape table written by the autotuner (JSON; path NULL:
  * $LUFQHE_SHAPE_TABLE, else shapes_gfx950.json next to the library).  An
  * entry is applied only if the candidate at its index still has the

@@ -6,6 +6,8 @@ The package directory name contains a hyphen, so import it with
 from .lucore import (  # noqa: F401
     ARITHS,
     POLICIES,
+    SHAPE_PINNED,
+    SHAPE_SMALL_BATCH,
     DetResult,
     LufqheError,
     MixedPlan,
@@ -26,7 +28,9 @@ from .lucore import (  # noqa: F401
     mc_split,
     pair_sum,
     read_matrices,
+    set_default_shape,
     set_shape,
     shape_count,
     shape_info,
+    uniform_shape,
 )

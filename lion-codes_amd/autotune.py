@@ -29,7 +29,7 @@ if str(_PKG.parent) not in sys.path:
 
 def time_shape(lc, A, res, policy: str, n: int, shape: int, reps: int) -> float:
     """Mean kernel time (ms) of `reps` launches with HIP events on the stream."""
-    assert lc.set_shape(policy, "fused", n, shape)
+    assert lc.set_shape(policy, "fused", n, shape | lc.SHAPE_PINNED)
     stream = torch.cuda.current_stream()
     lc.det_batched(A, policy=policy, out=res)
     torch.cuda.synchronize()
@@ -67,17 +67,21 @@ def tune(policies=("crout_ref", "abs"), ns=range(1, 65), target_mib: int = 256, 
             res = lc.alloc_result(cnt, n, dev)
             ref = None
             times = []
-            for shape in range(lc.shape_count(n)):
-                t = time_shape(lc, A, res, policy, n, shape, reps)
-                mant = res.mant.clone()
-                if ref is None:
-                    ref = mant
-                elif not torch.equal(torch.view_as_real(ref).view(torch.int64),
-                                     torch.view_as_real(mant).view(torch.int64)):
-                    raise RuntimeError(f"shape {shape} of n={n} ({policy}) differs from shape 0")
-                times.append(t)
+            keep = lc.get_shape(policy, "fused", n)
+            try:
+                for shape in range(lc.shape_count(n)):
+                    t = time_shape(lc, A, res, policy, n, shape, reps)
+                    mant = res.mant.clone()
+                    if ref is None:
+                        ref = mant
+                    elif not torch.equal(torch.view_as_real(ref).view(torch.int64),
+                                         torch.view_as_real(mant).view(torch.int64)):
+                        raise RuntimeError(f"shape {shape} of n={n} ({policy}) differs from shape 0")
+                    times.append(t)
+            finally:
+                lc.set_shape(policy, "fused", n, keep)
             best = min(range(len(times)), key=times.__getitem__)
-            lc.set_shape(policy, "fused", n, best)
+            lc.set_default_shape(policy, "fused", n, best)
             lanes, cols, waves = lc.shape_info(n, best)
             entries.append({"policy": policy, "n": n, "shape": best, "lanes": lanes,
                             "lane_cols": cols, "waves": waves, "count": cnt,

@@ -15,18 +15,19 @@ SmallLaunch g_small[kClassVariants][kMaxN + 1];
 
 namespace {
 thread_local hipError_t t_last_hip = hipSuccess;
-std::atomic<int> g_selected[kNumVariants][kMaxN + 1];  // zero-initialised: shape 0
+// zero-initialised: shape 0, not pinned
+std::atomic<int> g_selected[kNumVariants][kMaxN + 1];
+std::atomic<int> g_default[kNumVariants][kMaxN + 1];
 }
 
-constexpr int kPinned = 0x100;
+// The selected shape, with LUFQHE_SHAPE_PINNED where lufqhe_set_shape was given it.
+constexpr int kPinned = LUFQHE_SHAPE_PINNED;
 int selected_shape(int variant, int n) {
   return g_selected[variant][n].load(std::memory_order_relaxed) & ~kPinned;
 }
-void set_selected_shape(int variant, int n, int shape, bool pinned) {
-  g_selected[variant][n].store(shape | (pinned ? kPinned : 0), std::memory_order_relaxed);
-}
 bool shape_pinned(int variant, int n) {
-  return (g_selected[variant][n].load(std::memory_order_relaxed) & kPinned) != 0;
+  const int s = g_selected[variant][n].load(std::memory_order_relaxed);
+  return s != g_default[variant][n].load(std::memory_order_relaxed);
 }
 
 // The kernel a launch of (variant, n) uses: the selected shape if it is
@@ -41,21 +42,30 @@ int32_t hip_fail(hipError_t e) {
   return LUFQHE_ERROR_HIP;
 }
 
-extern thread_local bool t_loading_table;  // lufqhe_table.cpp
-
-// A uniform batch: the selected shape's kernel, or the small batch's.
-hipError_t launch_uniform(const KernelEntry& e, int variant, int n, const BatchArgs& args,
-                          int64_t blocks, hipStream_t stream) {
-  if (args.count <= kSmallMost && variant < kClassVariants && g_small[variant][n] &&
-      !shape_pinned(variant, n)) {
-    int dev = 0, cus = 0;
+// Whether a uniform batch runs the small batch's kernel, not the selected
+// shape's.  cus: compute units, or 0 to ask the current device if it matters.
+hipError_t small_route(int variant, int n, int64_t count, int cus, bool* small) {
+  *small = false;
+  if (count > kSmallMost || variant >= kClassVariants || !g_small[variant][n] ||
+      shape_pinned(variant, n))
+    return hipSuccess;
+  if (cus <= 0) {
+    int dev = 0;
     hipError_t err = hipGetDevice(&dev);
     if (err == hipSuccess)
       err = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (err != hipSuccess) return err;
-    if (small_batch(n, args.count, cus)) return g_small[variant][n](args, stream);
   }
-  return e.launch(args, blocks, stream);
+  *small = small_batch(n, count, cus);
+  return hipSuccess;
+}
+
+hipError_t launch_uniform(const KernelEntry& e, int variant, int n, const BatchArgs& args,
+                          int64_t blocks, hipStream_t stream) {
+  bool small = false;
+  const hipError_t err = small_route(variant, n, args.count, 0, &small);
+  if (err != hipSuccess) return err;
+  return small ? g_small[variant][n](args, stream) : e.launch(args, blocks, stream);
 }
 
 hipError_t launch_inplace_write(double2* A, int64_t count, int64_t stride, const double2* mant,
@@ -212,17 +222,35 @@ int32_t lufqhe_shape_info(int32_t n, int32_t shape, int32_t* lanes, int32_t* lan
 int32_t lufqhe_set_shape(int32_t policy, int32_t arith, int32_t n, int32_t shape) {
   const int v = variant_of(policy, arith);
   if (v < 0) return LUFQHE_ERROR_UNSUPPORTED;
-  if (n < 1 || n > kMaxN || shape < 0 || shape >= kMaxShapes) return LUFQHE_ERROR_INVALID_VALUE;
-  if (!g_kernels[v][n][shape].launch) return LUFQHE_ERROR_NOT_BUILT;
-  set_selected_shape(v, n, shape, !t_loading_table);
+  const int sh = shape & ~kPinned;
+  if (n < 1 || n > kMaxN || sh < 0 || sh >= kMaxShapes) return LUFQHE_ERROR_INVALID_VALUE;
+  if (!g_kernels[v][n][sh].launch) return LUFQHE_ERROR_NOT_BUILT;
+  g_selected[v][n].store(shape, std::memory_order_relaxed);
   return LUFQHE_SUCCESS;
+}
+
+int32_t lufqhe_set_default_shape(int32_t policy, int32_t arith, int32_t n, int32_t shape) {
+  if (shape < 0 || shape >= kMaxShapes) return LUFQHE_ERROR_INVALID_VALUE;  // no flag
+  const int32_t st = lufqhe_set_shape(policy, arith, n, shape);
+  if (st == LUFQHE_SUCCESS)
+    g_default[variant_of(policy, arith)][n].store(shape, std::memory_order_relaxed);
+  return st;
 }
 
 int32_t lufqhe_get_shape(int32_t policy, int32_t arith, int32_t n) {
   const int v = variant_of(policy, arith);
   if (v < 0 || n < 1 || n > kMaxN) return -1;
-  const int sh = selected_shape(v, n);
-  return g_kernels[v][n][sh].launch ? sh : 0;
+  const int sh = g_selected[v][n].load(std::memory_order_relaxed);
+  return g_kernels[v][n][sh & ~kPinned].launch ? sh : 0;
+}
+
+int32_t lufqhe_uniform_shape(int32_t policy, int32_t arith, int32_t n, int64_t batch,
+                             int32_t compute_units) {
+  const int v = variant_of(policy, arith);
+  if (v < 0 || n < 1 || n > kMaxN || batch < 1 || compute_units < 0) return -1;
+  bool small = false;
+  if (small_route(v, n, batch, compute_units, &small) != hipSuccess) return -1;
+  return small ? LUFQHE_SHAPE_SMALL_BATCH : lufqhe_get_shape(policy, arith, n) & ~kPinned;
 }
 
 int64_t lufqhe_det_inplace_workspace_bytes(int64_t count) {

@@ -17,17 +17,7 @@
 
 #include "../../include/lufqhe.h"
 
-namespace lufqhe {
-// set while a table is applied: its shapes are not pinned
-thread_local bool t_loading_table = false;
-}  // namespace lufqhe
-
 namespace {
-
-struct LoadingTable {
-  LoadingTable() { lufqhe::t_loading_table = true; }
-  ~LoadingTable() { lufqhe::t_loading_table = false; }
-};
 
 bool read_file(const std::string& path, std::string& out) {
   FILE* f = std::fopen(path.c_str(), "rb");
@@ -81,7 +71,6 @@ extern "C" int32_t lufqhe_load_shape_table(const char* path) {
   if (p == std::string::npos) return -1;
   p = text.find('[', p);
   if (p == std::string::npos) return -1;
-  const LoadingTable loading;
   int32_t applied = 0;
   int depth = 0;
   size_t start = 0;
@@ -106,7 +95,8 @@ extern "C" int32_t lufqhe_load_shape_table(const char* path) {
         if (lufqhe_shape_info(n, shape, &lanes, &cols, &waves) != LUFQHE_SUCCESS) continue;
         if (lanes != std::atoi(sl.c_str()) || cols != std::atoi(sc.c_str()) || waves != want_w)
           continue;
-        if (lufqhe_set_shape(policy, LUFQHE_ARITH_FUSED, n, shape) == LUFQHE_SUCCESS) ++applied;
+        if (lufqhe_set_default_shape(policy, LUFQHE_ARITH_FUSED, n, shape) == LUFQHE_SUCCESS)
+          ++applied;
       }
     } else if (c == ']' && depth == 0) {
       break;

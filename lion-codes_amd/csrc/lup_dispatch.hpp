@@ -50,10 +50,10 @@ struct KernelEntry {
 // shape of candidate_shape(); the reference-arithmetic variant only shape 0.
 extern KernelEntry g_kernels[kNumVariants][kMaxN + 1][kMaxShapes];
 
-// Shape chosen per (variant, n); 0 until the autotuner's table is applied.
-// A shape set by lufqhe_set_shape is pinned: it runs batches of every size.
+// Shape chosen per (variant, n); 0 until the autotuner's table is applied.  A
+// choice other than the default (the table's) is pinned: it runs uniform
+// batches of every size.
 int selected_shape(int variant, int n);
-void set_selected_shape(int variant, int n, int shape, bool pinned);
 bool shape_pinned(int variant, int n);
 
 // Class kernels (lup_class.hpp), one per fused variant (0: CROUT_REF, 1: ABS)

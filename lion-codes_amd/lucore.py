@@ -32,6 +32,8 @@ ERROR_NOT_BUILT = 4
 ERROR_OUT_OF_BUDGET = 5
 ERROR_IO = 6
 ERROR_TOO_LARGE = 7
+SHAPE_PINNED = 0x100       # in set_shape: the default shape for small batches too
+SHAPE_SMALL_BATCH = 0x200  # from uniform_shape: the kernel of small batches
 FILE_FORMATS = {"complex64": 0, "complex128": 1}
 
 _lib = None
@@ -86,6 +88,10 @@ def load() -> ctypes.CDLL:
                                       ctypes.POINTER(_i32)]
     lib.lufqhe_set_shape.restype = _i32
     lib.lufqhe_set_shape.argtypes = [_i32, _i32, _i32, _i32]
+    lib.lufqhe_set_default_shape.restype = _i32
+    lib.lufqhe_set_default_shape.argtypes = [_i32, _i32, _i32, _i32]
+    lib.lufqhe_uniform_shape.restype = _i32
+    lib.lufqhe_uniform_shape.argtypes = [_i32, _i32, _i32, _i64, _i32]
     lib.lufqhe_get_shape.restype = _i32
     lib.lufqhe_get_shape.argtypes = [_i32, _i32, _i32]
     lib.lufqhe_mixed_plan_create.restype = _i32
@@ -166,11 +172,23 @@ def shape_info(n: int, shape: int) -> tuple[int, int, int]:
 
 
 def set_shape(policy: str, arith: str, n: int, shape: int) -> bool:
+    """Select a shape; `shape | SHAPE_PINNED` runs the default one for small
+    batches too.  set_shape(get_shape()) restores a selection."""
     return load().lufqhe_set_shape(POLICIES[policy], ARITHS[arith], n, shape) == SUCCESS
+
+
+def set_default_shape(policy: str, arith: str, n: int, shape: int) -> bool:
+    """Select a shape and make it the default, as a shape table's entry does."""
+    return load().lufqhe_set_default_shape(POLICIES[policy], ARITHS[arith], n, shape) == SUCCESS
 
 
 def get_shape(policy: str, arith: str, n: int) -> int:
     return load().lufqhe_get_shape(POLICIES[policy], ARITHS[arith], n)
+
+
+def uniform_shape(policy: str, arith: str, n: int, batch: int, compute_units: int = 0) -> int:
+    """The shape a uniform batch runs now, or SHAPE_SMALL_BATCH."""
+    return load().lufqhe_uniform_shape(POLICIES[policy], ARITHS[arith], n, batch, compute_units)
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:

@@ -90,6 +90,46 @@ def test_shape_table_api(lc):
     assert lc.set_shape("crout_ref", "fused", 32, old)
 
 
+def test_selection_of_a_shape_round_trips(lc):
+    """get_shape, set_shape(x), set_shape(got) restores which kernel uniform
+    batches run, small ones included (256 compute units: 1024 matrices of
+    n = 17..32, 256 of n >= 49)."""
+    lib = lc.load()
+    for policy in ("crout_ref", "abs"):
+        for n in range(1, 65):
+            def routes(p=policy, n=n):
+                return [lc.uniform_shape(p, "fused", n, c, 256) for c in (1, limit, limit + 1)]
+            limit = 1024 if n <= 32 else 256
+            keep = lc.get_shape(policy, "fused", n)
+            small = lc.SHAPE_SMALL_BATCH if 17 <= n <= 32 or n >= 49 else keep
+            start = [small, small, keep]
+            assert routes() == start, (policy, n)
+            for s in range(lc.shape_count(n)):
+                assert lc.set_shape(policy, "fused", n, s)
+                assert lc.get_shape(policy, "fused", n) == s
+                assert routes() == (start if s == keep else [s, s, s]), (policy, n, s)
+                assert lc.set_shape(policy, "fused", n, s | lc.SHAPE_PINNED)
+                assert routes() == [s, s, s], (policy, n, s)
+                got = lc.get_shape(policy, "fused", n)  # a pinned selection round trips too
+                assert lc.set_shape(policy, "fused", n, 0) and lc.set_shape(policy, "fused", n, got)
+                assert routes() == [s, s, s], (policy, n, s)
+                assert lc.set_shape(policy, "fused", n, keep)
+                assert routes() == start, (policy, n, s)
+            # another default: its own round trip
+            s = lc.shape_count(n) - 1
+            assert lc.set_default_shape(policy, "fused", n, s)
+            assert routes() == [s if small == keep else small] * 2 + [s]
+            assert lc.set_default_shape(policy, "fused", n, keep)
+            assert routes() == start
+    for fn in (lib.lufqhe_set_shape, lib.lufqhe_set_default_shape):
+        assert fn(0, 0, 32, -1) == 1 and fn(0, 0, 32, 7) == 1 and fn(0, 0, 32, 0x200) == 1
+        assert fn(0, 1, 32, 1) == 4 and fn(1, 1, 32, 0) == 2
+    assert lib.lufqhe_set_default_shape(0, 0, 32, 0x100) == 1   # a default is never pinned
+    assert lib.lufqhe_uniform_shape(0, 1, 32, 10, 256) == 0     # reference arithmetic: its one shape
+    for bad in ((9, 0, 32, 10, 256), (0, 0, 0, 10, 256), (0, 0, 32, 0, 256), (0, 0, 32, 10, -1)):
+        assert lib.lufqhe_uniform_shape(*bad) == -1
+
+
 def test_fqhe_argument_validation(lc):
     lib = lc.load()
     args = (None, None, None, None, None, None, 0, 0, None)

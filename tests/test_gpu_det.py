@@ -360,7 +360,8 @@ def test_every_launch_shape_bit_exact(lc, orc, wl, dev, n):
         keep = lc.get_shape(policy, "fused", n)
         try:
             for shape in range(lc.shape_count(n)):
-                assert lc.set_shape(policy, "fused", n, shape)
+                assert lc.set_shape(policy, "fused", n, shape | lc.SHAPE_PINNED)
+                assert lc.uniform_shape(policy, "fused", n, len(A)) == shape
                 assert_same(run(lc, A, dev, policy, "fused"), o, n, (policy, shape))
         finally:
             lc.set_shape(policy, "fused", n, keep)

@@ -50,7 +50,7 @@ def test_fused_build_equals_materialised(lc, orc, wl, dev, n):
     old = lc.get_shape("crout_ref", "fused", n)
     try:
         for sh in range(lc.shape_count(n)):
-            lc.set_shape("crout_ref", "fused", n, sh)
+            assert lc.set_shape("crout_ref", "fused", n, sh | lc.SHAPE_PINNED)
             same(lc.fqhe_det(z), ref)
     finally:
         lc.set_shape("crout_ref", "fused", n, old)

@@ -29,7 +29,7 @@ def check(lc, orc, dev, A):
         keep = lc.get_shape(policy, "fused", n)
         try:
             for shape in range(lc.shape_count(n)):
-                assert lc.set_shape(policy, "fused", n, shape)
+                assert lc.set_shape(policy, "fused", n, shape | lc.SHAPE_PINNED)
                 r = lc.det_batched(d, policy=policy, pivots=True)
                 torch.cuda.synchronize()
                 what = (n, policy, shape)
@@ -89,7 +89,6 @@ def test_criteria_outside_the_corrected_range(lc, orc, wl, dev, n):
 def test_small_batches(lc, orc, wl, dev, n, limit):
     """The low-latency kernels of batches that leave SIMDs idle, on both sides
     of the line where they end (256 compute units), in a padded layout."""
-    lc.apply_shape_table()  # a table's shapes are not pinned
     base = wl.gaussian_np(64, n, seed=900 + n)
     base[0] = np.round(base[0])
     base[1] = np.round(base[1].real)
@@ -97,7 +96,10 @@ def test_small_batches(lc, orc, wl, dev, n, limit):
     base[3] *= 2.0 ** 980
     for policy in ("crout_ref", "abs"):
         o = orc.mirror(base, policy, "fused")
+        keep = lc.get_shape(policy, "fused", n)
         for count in (1, 2, 64, limit, limit + 1):
+            want = lc.SHAPE_SMALL_BATCH if count <= limit else keep
+            assert lc.uniform_shape(policy, "fused", n, count) == want
             idx = np.arange(count) % 64
             A = torch.zeros(count, n, n + 3, dtype=torch.complex128, device=dev)
             A[:, :, :n] = torch.from_numpy(base[idx]).to(dev)
@@ -115,21 +117,36 @@ def test_small_batches(lc, orc, wl, dev, n, limit):
 def test_small_batches_built_on_the_device(lc, wl, dev, n):
     """The same kernels building their matrices from permuted positions (one
     permutation entry out of range) equal the pinned shape's."""
-    lc.apply_shape_table()
     rng = np.random.default_rng(n)
     z = torch.from_numpy(wl.fqhe_positions(n, rng)[None, :]).to(dev)
     perm = np.argsort(rng.random((9, n)), axis=1).astype(np.uint8)
     perm[4, n - 1] = n
     p = torch.from_numpy(perm).to(dev)
+    assert lc.uniform_shape("crout_ref", "fused", n, 9) == lc.SHAPE_SMALL_BATCH
     small = lc.fqhe_det(z, row_perm=p, count=9, pivots=True)
     sh = lc.get_shape("crout_ref", "fused", n)
     try:
-        assert lc.set_shape("crout_ref", "fused", n, sh)  # pinned
+        assert lc.set_shape("crout_ref", "fused", n, sh | lc.SHAPE_PINNED)
+        assert lc.uniform_shape("crout_ref", "fused", n, 9) == sh
         big = lc.fqhe_det(z, row_perm=p, count=9, pivots=True)
     finally:
-        lc.apply_shape_table()
+        lc.set_shape("crout_ref", "fused", n, sh)
     torch.cuda.synchronize()
     assert small.info.cpu().tolist() == big.info.cpu().tolist()
     assert small.info[4].item() == -1000
     assert torch.equal(small.piv, big.piv) and torch.equal(small.exp, big.exp)
     assert same(small.mant.cpu().numpy(), big.mant.cpu().numpy())
+
+
+def test_tuning_leaves_the_small_batch_kernels_on(lc, dev):
+    """The tuner pins each shape while it times it, small counts included, and
+    leaves its choice as the default."""
+    from importlib import import_module
+    tune = import_module("lion-codes_amd.autotune").tune
+    try:
+        table = tune(ns=[20, 32, 64], reps=1, count=96, log=lambda m: None)
+        for e in table["entries"]:
+            assert lc.get_shape(e["policy"], "fused", e["n"]) == e["shape"]
+            assert lc.uniform_shape(e["policy"], "fused", e["n"], 48) == lc.SHAPE_SMALL_BATCH
+    finally:
+        lc.apply_shape_table()
