@@ -149,10 +149,18 @@ def apply_shape_table(path: Path | None = None) -> int:
     p = Path(path) if path is not None else SHAPE_TABLE
     if not p.exists():
         return 0
-    # an entry applies only to the candidate it was measured on
-    applied = load().lufqhe_load_shape_table(str(p).encode())
-    if applied < 0:
-        raise ValueError(f"{p} is not a shape table")
+    import json
+    table = json.loads(p.read_text())
+    applied = 0
+    for e in table.get("entries", []):
+        n, sh = int(e["n"]), int(e["shape"])
+        # an entry applies only to the candidate it was measured on
+        if not 0 <= sh < shape_count(n):
+            continue
+        if shape_info(n, sh) != (e["lanes"], e["lane_cols"], e.get("waves", 1)):
+            continue
+        if set_default_shape(e["policy"], "fused", n, sh):
+            applied += 1
     return applied
 
 

@@ -90,6 +90,34 @@ def test_shape_table_api(lc):
     assert lc.set_shape("crout_ref", "fused", 32, old)
 
 
+def test_package_reads_a_shape_table_as_json(lc, tmp_path):
+    """apply_shape_table reads any valid JSON table, and refuses a damaged one
+    whole instead of applying what comes before the damage."""
+    import json
+    from importlib import import_module
+    entries = json.loads(import_module("lion-codes_amd.lucore").SHAPE_TABLE.read_text())["entries"]
+    first = next(e for e in entries if e["shape"] != 0)
+    text = json.dumps({"note": {"entries": [1]}, "entries": [first] + entries[:3]},
+                      separators=(", ", " :\r "))
+    p = tmp_path / "t.json"
+
+    def apply(s):
+        p.write_text(s, newline="")
+        return lc.apply_shape_table(p)
+    assert lc.apply_shape_table(tmp_path / "missing.json") == 0
+    assert apply("{}") == 0 and apply('{"entries": []}') == 0
+    assert apply(text) == 4
+    where = (first["policy"], "fused", first["n"])
+    assert lc.get_shape(*where) == first["shape"] and lc.set_default_shape(*where, 0)
+    for bad in ("", text[:-20], text + "}"):
+        with pytest.raises(json.JSONDecodeError):
+            apply(bad)
+    assert lc.get_shape(*where) == 0
+    with pytest.raises(KeyError):
+        apply(json.dumps({"entries": [{k: v for k, v in entries[0].items() if k != "n"}]}))
+    lc.apply_shape_table()
+
+
 def test_selection_of_a_shape_round_trips(lc):
     """get_shape, set_shape(x), set_shape(got) restores which kernel uniform
     batches run, small ones included (256 compute units: 1024 matrices of
