@@ -108,6 +108,11 @@ int32_t lufqhe_det_batched(const void *d_A, int64_t batch, int32_t n,
 int32_t lufqhe_shape_count(int32_t n);
 int32_t lufqhe_shape_info(int32_t n, int32_t shape, int32_t *lanes,
                           int32_t *lane_cols, int32_t *min_waves);
+/* Which kernel a shape is of: two shapes of one n can be alike in
+ * lufqhe_shape_info and differ in this.  -1 for invalid arguments. */
+#define LUFQHE_KERNEL_VECTOR 0
+#define LUFQHE_KERNEL_PANEL 1
+int32_t lufqhe_shape_kernel(int32_t n, int32_t shape);
 int32_t lufqhe_set_shape(int32_t policy, int32_t arith, int32_t n,
                          int32_t shape);
 /* Selects a shape and makes it the default, as a table's entry does. */
@@ -123,8 +128,9 @@ int32_t lufqhe_uniform_shape(int32_t policy, int32_t arith, int32_t n,
 /* Applies a shape table written by the autotuner (JSON; path NULL:
  * $LUFQHE_SHAPE_TABLE, else shapes_gfx950.json next to the library).  An
  * entry is applied only if the candidate at its index still has the
- * recorded (lanes, lane_cols, waves).  Returns the number of entries
- * applied, or -1 if the file cannot be read or holds no entry list. */
+ * recorded (lanes, lane_cols, waves) and kernel ("vector" or "panel"; an
+ * entry without it was measured on a vector kernel).  Returns the number of
+ * entries applied, or -1 if the file cannot be read or holds no entry list. */
 int32_t lufqhe_load_shape_table(const char *path);
 
 /* Bytes of device workspace lufqhe_det_inplace needs for `count` matrices

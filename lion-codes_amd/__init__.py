@@ -32,5 +32,6 @@ from .lucore import (  # noqa: F401
     set_shape,
     shape_count,
     shape_info,
+    shape_kernel,
     uniform_shape,
 )

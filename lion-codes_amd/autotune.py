@@ -84,10 +84,12 @@ def tune(policies=("crout_ref", "abs"), ns=range(1, 65), target_mib: int = 256, 
             lc.set_default_shape(policy, "fused", n, best)
             lanes, cols, waves = lc.shape_info(n, best)
             entries.append({"policy": policy, "n": n, "shape": best, "lanes": lanes,
-                            "lane_cols": cols, "waves": waves, "count": cnt,
+                            "lane_cols": cols, "waves": waves,
+                            "kernel": lc.shape_kernel(n, best), "count": cnt,
                             "us_per_launch": [round(t * 1e3, 2) for t in times],
                             "ns_per_det": round(times[best] * 1e6 / cnt, 3)})
-            log(f"{policy:9s} n={n:2d} shape={best} (L={lanes}, CG={cols}, waves={waves}) "
+            log(f"{policy:9s} n={n:2d} shape={best} (L={lanes}, CG={cols}, waves={waves}, "
+                f"{lc.shape_kernel(n, best)}) "
                 f"times(us)={[round(t * 1e3, 1) for t in times]}")
             del A, res
     props = torch.cuda.get_device_properties(0)

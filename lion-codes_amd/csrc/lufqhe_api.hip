@@ -219,6 +219,13 @@ int32_t lufqhe_shape_info(int32_t n, int32_t shape, int32_t* lanes, int32_t* lan
   return LUFQHE_SUCCESS;
 }
 
+int32_t lufqhe_shape_kernel(int32_t n, int32_t shape) {
+  if (n < 1 || n > kMaxN || shape < 0 || shape >= kMaxShapes) return -1;
+  const KernelEntry& e = g_kernels[0][n][shape];
+  if (!e.launch) return -1;
+  return e.shape.panel ? LUFQHE_KERNEL_PANEL : LUFQHE_KERNEL_VECTOR;
+}
+
 int32_t lufqhe_set_shape(int32_t policy, int32_t arith, int32_t n, int32_t shape) {
   const int v = variant_of(policy, arith);
   if (v < 0) return LUFQHE_ERROR_UNSUPPORTED;

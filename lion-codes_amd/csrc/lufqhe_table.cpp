@@ -2,11 +2,13 @@
 //
 // lion-codes_amd/autotune.py writes one JSON file per device kind:
 //   {"device": ..., "entries": [{"policy": "crout_ref", "n": 32, "shape": 0,
-//     "lanes": 32, "lane_cols": 2, "waves": 1, ...}, ...]}
+//     "lanes": 32, "lane_cols": 2, "waves": 1,
+//     "kernel": "vector", ...}, ...]}
 // lufqhe_load_shape_table selects each entry's shape for the fused
 // arithmetic, so C and C++ callers (LUCoreGPU::CALL included) run the tuned
 // kernels without the Python package.  An entry applies only while the
-// compiled candidate at that index still has the recorded geometry.
+// compiled candidate at that index still has the recorded geometry and kernel
+// (no "kernel": written before there were panel kernels, so "vector").
 #include <dlfcn.h>
 
 #include <cctype>
@@ -87,7 +89,7 @@ extern "C" int32_t lufqhe_load_shape_table(const char* path) {
                                               : -1;
         const std::string sn = field(obj, "n"), ss = field(obj, "shape");
         const std::string sl = field(obj, "lanes"), sc = field(obj, "lane_cols");
-        const std::string sw = field(obj, "waves");
+        const std::string sw = field(obj, "waves"), sk = field(obj, "kernel");
         if (policy < 0 || sn.empty() || ss.empty() || sl.empty() || sc.empty()) continue;
         const int n = std::atoi(sn.c_str()), shape = std::atoi(ss.c_str());
         const int want_w = sw.empty() ? 1 : std::atoi(sw.c_str());
@@ -95,6 +97,10 @@ extern "C" int32_t lufqhe_load_shape_table(const char* path) {
         if (lufqhe_shape_info(n, shape, &lanes, &cols, &waves) != LUFQHE_SUCCESS) continue;
         if (lanes != std::atoi(sl.c_str()) || cols != std::atoi(sc.c_str()) || waves != want_w)
           continue;
+        const int32_t want_k = sk.empty() || sk == "vector" ? LUFQHE_KERNEL_VECTOR
+                               : sk == "panel"              ? LUFQHE_KERNEL_PANEL
+                                                            : -2;
+        if (lufqhe_shape_kernel(n, shape) != want_k) continue;
         if (lufqhe_set_default_shape(policy, LUFQHE_ARITH_FUSED, n, shape) == LUFQHE_SUCCESS)
           ++applied;
       }

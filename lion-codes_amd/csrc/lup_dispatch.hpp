@@ -34,6 +34,7 @@ struct KernelShape {
   int lane_cols;
   int waves_per_block;
   int min_waves;  // waves per SIMD the register allocation allows at least
+  bool panel;     // lup_panel_kernel, else lup_det_kernel
 };
 
 // Launches the (variant, n) kernel on `blocks` workgroups.

@@ -52,7 +52,7 @@ void register_shape() {
                   "the panel kernel's geometry");
     KernelEntry& e = g_kernels[LUFQHE_VARIANT][N][SH];
     e.launch = &launch<N, SH>;
-    e.shape = KernelShape{sh.lanes, sh.lane_cols, kWavesPerBlock, sh.waves};
+    e.shape = KernelShape{sh.lanes, sh.lane_cols, kWavesPerBlock, sh.waves, sh.panel};
     e.kernel = reinterpret_cast<const void*>(kernel_of<N, SH>());
   }
 }

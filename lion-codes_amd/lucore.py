@@ -86,6 +86,8 @@ def load() -> ctypes.CDLL:
     lib.lufqhe_shape_info.restype = _i32
     lib.lufqhe_shape_info.argtypes = [_i32, _i32, ctypes.POINTER(_i32), ctypes.POINTER(_i32),
                                       ctypes.POINTER(_i32)]
+    lib.lufqhe_shape_kernel.restype = _i32
+    lib.lufqhe_shape_kernel.argtypes = [_i32, _i32]
     lib.lufqhe_set_shape.restype = _i32
     lib.lufqhe_set_shape.argtypes = [_i32, _i32, _i32, _i32]
     lib.lufqhe_set_default_shape.restype = _i32
@@ -159,6 +161,9 @@ def apply_shape_table(path: Path | None = None) -> int:
             continue
         if shape_info(n, sh) != (e["lanes"], e["lane_cols"], e.get("waves", 1)):
             continue
+        # a table without "kernel" is older than the panel kernels
+        if shape_kernel(n, sh) != e.get("kernel", "vector"):
+            continue
         if set_default_shape(e["policy"], "fused", n, sh):
             applied += 1
     return applied
@@ -177,6 +182,15 @@ def shape_info(n: int, shape: int) -> tuple[int, int, int]:
     if st != SUCCESS:
         raise LufqheError("lufqhe_shape_info", st)
     return lanes.value, cols.value, waves.value
+
+
+def shape_kernel(n: int, shape: int) -> str:
+    """Which kernel candidate `shape` is of: "vector" (lup_kernel.hpp) or
+    "panel" (lup_panel.hpp)."""
+    k = load().lufqhe_shape_kernel(n, shape)
+    if k < 0:
+        raise LufqheError("lufqhe_shape_kernel", ERROR_INVALID_VALUE)
+    return "panel" if k else "vector"
 
 
 def set_shape(policy: str, arith: str, n: int, shape: int) -> bool:

@@ -23,6 +23,7 @@ int32_t lufqhe_shape_info(int32_t n, int32_t shape, int32_t* lanes, int32_t* col
   if (waves) *waves = 1;
   return LUFQHE_SUCCESS;
 }
+int32_t lufqhe_shape_kernel(int32_t n, int32_t) { return n > 24; }
 int32_t lufqhe_set_default_shape(int32_t, int32_t, int32_t, int32_t) { return LUFQHE_SUCCESS; }
 const char* lufqhe_status_string(int32_t) { return "stub"; }
 }

@@ -191,7 +191,23 @@ def test_shape_table_loads_from_c(lc, tmp_path):
         p = tmp_path / "t.json"
         p.write_text(json.dumps({"entries": [bad]}))
         assert lib.lufqhe_load_shape_table(str(p).encode()) == 0
+        # and so is one measured on another kernel of the same geometry, by
+        # both readers: no "kernel" means a vector kernel
+        kinds = {(n, lc.shape_kernel(n, 0), lc.shape_kernel(n, lc.shape_count(n) - 1))
+                 for n in (16, 20, 52)}
+        assert kinds == {(16, "vector", "vector"), (20, "vector", "panel"), (52, "panel", "panel")}
+        for n, sh in ((16, 0), (20, 0), (20, 3), (52, 0), (52, 1)):
+            lanes, cols, waves = lc.shape_info(n, sh)
+            e = {"policy": "abs", "n": n, "shape": sh, "lanes": lanes, "lane_cols": cols,
+                 "waves": waves}
+            for kind in (None, "vector", "panel", "other"):
+                p.write_text(json.dumps({"entries": [e if kind is None else dict(e, kernel=kind)]}))
+                want = int((kind or "vector") == lc.shape_kernel(n, sh))
+                assert lib.lufqhe_load_shape_table(str(p).encode()) == want, (n, sh, kind)
+                assert lc.apply_shape_table(p) == want, (n, sh, kind)
+        assert lib.lufqhe_shape_kernel(16, 2) == -1 and lib.lufqhe_shape_kernel(65, 0) == -1
         assert lib.lufqhe_load_shape_table(str(tmp_path / "missing.json").encode()) == -1
     finally:
+        lc.apply_shape_table()
         for (pol, n), sh in saved.items():
             lc.set_shape(pol, "fused", n, sh)
