@@ -371,9 +371,17 @@ int32_t lufqhe_mc_lu_run(const void *h_matrices, int64_t nelem, int32_t n,
  * (seed, request), so records are bit-identical for any rate or batching.
  * Results per request go to `records` (may be NULL); the walkers keep their
  * final configurations (lufqhe_server_reset restores the initial ones).
- * The run allocates its batch buffers (hipMalloc, pinned host memory) and
- * frees them before returning.  A server runs on the device that was current
- * when it was created (else LUFQHE_ERROR_INVALID_VALUE). */
+ * A run allocates its batch buffers (hipMalloc, pinned host memory, streams)
+ * and leaves them to the server's next run, which takes them if its
+ * max_batch_requests, max_inflight and max_batch_dets are the same and frees
+ * them otherwise.  A process keeps at most 256 MiB in 16 such sets, whatever
+ * the number of servers: the oldest set makes room, and a run with more frees
+ * its buffers before returning.  Kept buffers are outside every hbm_budget; an
+ * allocation of this library (servers, plans, the Monte Carlo loop, the file
+ * reader) that finds no device memory frees them all and tries again, and
+ * lufqhe_server_release and lufqhe_server_destroy free them.  One run at a time
+ * per server; different servers may run at once.  A server runs on the device
+ * that was current when it was created (else LUFQHE_ERROR_INVALID_VALUE). */
 #define LUFQHE_SERVE_MAX_INFLIGHT 8
 
 typedef struct lufqhe_server lufqhe_server;
@@ -411,6 +419,10 @@ int32_t lufqhe_server_create(int32_t walkers, const int32_t *h_walker_n,
                              int32_t policy, lufqhe_server **server);
 int32_t lufqhe_server_destroy(lufqhe_server *server);
 int32_t lufqhe_server_reset(lufqhe_server *server);
+/* Frees the buffers kept for the server's next run (every server's if NULL), or
+ * tells how many bytes they hold, device and pinned. */
+int32_t lufqhe_server_release(lufqhe_server *server);
+int64_t lufqhe_server_kept_bytes(const lufqhe_server *server);
 /* Walker w's n and (if h_z) its current configuration (n complex128). */
 int32_t lufqhe_server_walker(const lufqhe_server *server, int32_t walker,
                              int32_t *n, void *h_z);

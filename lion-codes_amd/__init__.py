@@ -28,6 +28,7 @@ from .lucore import (  # noqa: F401
     mc_split,
     pair_sum,
     read_matrices,
+    release_server_buffers,
     set_default_shape,
     set_shape,
     shape_count,

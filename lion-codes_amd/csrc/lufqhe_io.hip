@@ -25,6 +25,7 @@
 
 namespace lufqhe {
 int32_t hip_fail(hipError_t e);
+hipError_t device_malloc(void** p, size_t bytes);
 }  // namespace lufqhe
 
 using namespace lufqhe;
@@ -114,7 +115,7 @@ int32_t lufqhe_read_matrices(const char* path, int32_t format, int64_t count, in
   for (int b = 0; b < 2 && err == hipSuccess; ++b) {
     err = hipHostMalloc(&s.host[b], (size_t)kStageBytes, 0);
     if (err == hipSuccess && format == LUFQHE_FILE_COMPLEX64)
-      err = hipMalloc(&s.dev[b], (size_t)kStageBytes);
+      err = device_malloc((void**)&s.dev[b], (size_t)kStageBytes);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&s.done[b], hipEventDisableTiming);
   }
   if (err != hipSuccess) return hip_fail(err);

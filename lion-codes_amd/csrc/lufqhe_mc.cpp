@@ -21,6 +21,7 @@
 
 namespace lufqhe {
 int32_t hip_fail(hipError_t e);  // lufqhe_api.hip
+hipError_t device_malloc(void** p, size_t bytes);  // lufqhe_serve.hip
 }
 
 namespace {
@@ -90,12 +91,12 @@ extern "C" int32_t lufqhe_mc_lu_run(const void* h_matrices, int64_t nelem, int32
   hipError_t err = hipStreamCreateWithFlags(&b.stream, hipStreamNonBlocking);
   if (err == hipSuccess) err = hipEventCreate(&b.ev0);
   if (err == hipSuccess) err = hipEventCreate(&b.ev1);
-  if (err == hipSuccess && ng > 0) err = hipMalloc(&b.d_A, gpu_bytes);
+  if (err == hipSuccess && ng > 0) err = lufqhe::device_malloc((void**)&b.d_A, gpu_bytes);
   const int64_t ws_inplace = lufqhe_det_inplace_workspace_bytes(ng);
   const int64_t ws_sum = lufqhe_pair_sum_workspace_bytes();
   if (err == hipSuccess && ng > 0)
-    err = hipMalloc(&b.d_work, (size_t)(ws_inplace > ws_sum ? ws_inplace : ws_sum));
-  if (err == hipSuccess) err = hipMalloc(&b.d_sum, sizeof(Cplx));
+    err = lufqhe::device_malloc((void**)&b.d_work, (size_t)(ws_inplace > ws_sum ? ws_inplace : ws_sum));
+  if (err == hipSuccess) err = lufqhe::device_malloc((void**)&b.d_sum, sizeof(Cplx));
   if (err == hipSuccess) err = hipHostMalloc(reinterpret_cast<void**>(&b.h_sum), sizeof(Cplx));
   if (err == hipSuccess && ng > 0) err = hipHostMalloc(&b.h_stage, gpu_bytes);
   if (err != hipSuccess) return lufqhe::hip_fail(err);

@@ -35,6 +35,7 @@ namespace lufqhe {
 int32_t hip_fail(hipError_t e);
 const KernelEntry& entry_for(int variant, int n);
 int64_t plain_blocks(const KernelEntry& e, int64_t count);
+hipError_t device_malloc(void** p, size_t bytes);
 }  // namespace lufqhe
 
 using namespace lufqhe;
@@ -237,7 +238,8 @@ int32_t lufqhe_mixed_plan_create(const int32_t* h_n, const int64_t* h_offs, int6
   std::sort(p->buckets.begin(), p->buckets.end(),
             [](const auto& a, const auto& b) { return a.cost > b.cost; });
 
-  if (err == hipSuccess && count > 0) err = hipMalloc(&p->d_tables, tables.size() * sizeof(int64_t));
+  if (err == hipSuccess && count > 0) 
+    err = device_malloc((void**)&p->d_tables, tables.size() * sizeof(int64_t));
   if (err == hipSuccess && count > 0)
     err = hipMemcpy(p->d_tables, tables.data(), tables.size() * sizeof(int64_t),
                     hipMemcpyHostToDevice);

@@ -34,12 +34,12 @@
 #include <cstring>
 #include <deque>
 #include <memory>
-#include <mutex>
 #include <new>
 #include <thread>
 #include <vector>
 
 #include "../../include/lufqhe.h"
+#include "kept_pool.hpp"
 #include "lup_dispatch.hpp"
 #include "scaled_sum.hpp"
 
@@ -47,6 +47,7 @@ namespace lufqhe {
 int32_t hip_fail(hipError_t e);
 const KernelEntry& entry_for(int variant, int n);
 int64_t plain_blocks(const KernelEntry& e, int64_t count);
+hipError_t device_malloc(void** p, size_t bytes);
 }  // namespace lufqhe
 
 using namespace lufqhe;
@@ -255,7 +256,36 @@ struct RunBuffers {
   }
 };
 
+// The buffers of each server's last run, for its next one with the same
+// limits: allocating and freeing them (pinned memory, streams, device blocks)
+// took 2 of the 5 ms of a 384-request run.  The limit holds one set of the
+// package's default limits (four batches of 2^20 determinants, 177 MiB); it is
+// 0.09% of the device's memory, and larger sets are freed when their run ends.
+// Never destroyed: its sets must not outlive the HIP runtime.
+constexpr int64_t kKeepMost = int64_t{256} << 20;
+KeptPool<RunBuffers>& kept_buffers() {
+  static KeptPool<RunBuffers>& pool = *new KeptPool<RunBuffers>(kKeepMost);
+  return pool;
+}
+
+// alloc() again without the kept buffers if the memory they hold is missing.
+template <class F>
+hipError_t alloc_or_release(F alloc) {
+  hipError_t err = alloc();
+  if (err == hipErrorOutOfMemory && kept_buffers().release(nullptr)) {
+    (void)hipGetLastError();  // not the next launch's error
+    err = alloc();
+  }
+  return err;
+}
+
 }  // namespace
+
+namespace lufqhe {
+hipError_t device_malloc(void** p, size_t bytes) {
+  return alloc_or_release([&] { return hipMalloc(p, bytes); });
+}
+}  // namespace lufqhe
 
 // ---------------------------------------------------------------- server
 struct lufqhe_server {
@@ -270,14 +300,9 @@ struct lufqhe_server {
   double2* d_walker_z = nullptr;      // [walkers][64]
   uint8_t* d_perm = nullptr;          // [walkers][perms][64]
   int64_t resident_bytes = 0;
-  // The buffers of the last run, for one with the same limits: allocating and
-  // freeing them (pinned memory, streams, device blocks) took 2 of the 5 ms of
-  // a 384-request run.  At most one set, freed with the server or by a run with
-  // other limits; runs that overlap allocate their own.
-  std::mutex mu;
-  std::unique_ptr<RunBuffers> kept;
 
   ~lufqhe_server() {
+    kept_buffers().release(this);
     if (d_walker_z) (void)hipFree(d_walker_z);
     if (d_perm) (void)hipFree(d_perm);
   }
@@ -308,6 +333,9 @@ struct Run {
   lufqhe_serve_config cfg;
   int64_t arena_bytes = 0;
   std::unique_ptr<RunBuffers> buf;
+  int64_t pinned_bytes() const {
+    return buf->inflight * buf->R * (int64_t)(sizeof(ReqDesc) + sizeof(double2) + sizeof(int32_t));
+  }
   std::vector<int32_t> free_slots;
   // walker state
   std::vector<int32_t> commit;   // slot with the accepted, uncommitted configuration
@@ -447,8 +475,8 @@ int32_t lufqhe_server_create(int32_t walkers, const int32_t* h_walker_n, int32_t
   if (err == hipSuccess)
     err = hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, s->device);
   const size_t zb = s->z0.size() * sizeof(double2);
-  if (err == hipSuccess) err = hipMalloc(&s->d_walker_z, zb);
-  if (err == hipSuccess) err = hipMalloc(&s->d_perm, perm.size());
+  if (err == hipSuccess) err = device_malloc((void**)&s->d_walker_z, zb);
+  if (err == hipSuccess) err = device_malloc((void**)&s->d_perm, perm.size());
   if (err == hipSuccess) err = hipMemcpy(s->d_walker_z, s->z0.data(), zb, hipMemcpyHostToDevice);
   if (err == hipSuccess) err = hipMemcpy(s->d_perm, perm.data(), perm.size(), hipMemcpyHostToDevice);
   if (err != hipSuccess) {
@@ -471,6 +499,13 @@ int32_t lufqhe_server_reset(lufqhe_server* s) {
                                    hipMemcpyHostToDevice);
   return err == hipSuccess ? LUFQHE_SUCCESS : hip_fail(err);
 }
+
+int32_t lufqhe_server_release(lufqhe_server* s) {
+  kept_buffers().release(s);
+  return LUFQHE_SUCCESS;
+}
+
+int64_t lufqhe_server_kept_bytes(const lufqhe_server* s) { return kept_buffers().bytes(s); }
 
 int32_t lufqhe_server_walker(const lufqhe_server* s, int32_t walker, int32_t* n, void* h_z) {
   if (!s || walker < 0 || walker >= s->walkers) return LUFQHE_ERROR_INVALID_VALUE;
@@ -508,15 +543,14 @@ int32_t lufqhe_server_run(lufqhe_server* s, const lufqhe_serve_config* cfg,
   run.s = s;
   run.cfg = *cfg;
   run.arena_bytes = arena;
-  {
-    std::lock_guard<std::mutex> lock(s->mu);
-    if (s->kept && s->kept->fits(*cfg)) run.buf = std::move(s->kept);
-    s->kept.reset();
-  }
+  run.buf = kept_buffers().take(s);
+  if (run.buf && !run.buf->fits(*cfg)) run.buf.reset();
   if (!run.buf) {
-    run.buf.reset(new (std::nothrow) RunBuffers());
-    if (!run.buf) return LUFQHE_ERROR_HIP;
-    err = run.buf->alloc(*cfg, s->walkers);
+    err = alloc_or_release([&] {
+      run.buf.reset();  // what a first try got
+      run.buf.reset(new (std::nothrow) RunBuffers());
+      return run.buf ? run.buf->alloc(*cfg, s->walkers) : hipErrorOutOfMemory;
+    });
     if (err != hipSuccess) return hip_fail(err);
   }
   for (int64_t i = run.buf->nslots - 1; i >= 0; --i) run.free_slots.push_back((int32_t)i);
@@ -696,11 +730,9 @@ int32_t lufqhe_server_run(lufqhe_server* s, const lufqhe_serve_config* cfg,
     }
   }
   if (err != hipSuccess) return hip_fail(err);
-  {
-    // every batch has completed and the last commit was waited for
-    std::lock_guard<std::mutex> lock(s->mu);
-    if (!s->kept) s->kept = std::move(run.buf);
-  }
+  // every batch has completed and the last commit was waited for
+  const int64_t held = run.arena_bytes + run.pinned_bytes();
+  kept_buffers().put(s, std::move(run.buf), held);
 
   if (stats) {
     std::vector<double> lat(latency);

@@ -113,6 +113,10 @@ def load() -> ctypes.CDLL:
     lib.lufqhe_server_destroy.argtypes = [_vp]
     lib.lufqhe_server_reset.restype = _i32
     lib.lufqhe_server_reset.argtypes = [_vp]
+    lib.lufqhe_server_release.restype = _i32
+    lib.lufqhe_server_release.argtypes = [_vp]
+    lib.lufqhe_server_kept_bytes.restype = _i64
+    lib.lufqhe_server_kept_bytes.argtypes = [_vp]
     lib.lufqhe_server_walker.restype = _i32
     lib.lufqhe_server_walker.argtypes = [_vp, _i32, ctypes.POINTER(_i32), _vp]
     lib.lufqhe_server_perms.restype = _i32
@@ -546,6 +550,15 @@ class Server:
         if st != SUCCESS:
             raise LufqheError("lufqhe_server_reset", st)
 
+    def release(self) -> None:
+        """Free the buffers kept for the next run."""
+        if self._h:
+            _lib.lufqhe_server_release(self._h)
+
+    def kept_bytes(self) -> int:
+        """Device and pinned bytes kept for the next run."""
+        return _lib.lufqhe_server_kept_bytes(self._h) if self._h else 0
+
     def walker(self, w: int):
         """Walker w's current configuration (complex128 [n])."""
         import numpy as np
@@ -575,6 +588,11 @@ class Server:
             self.close()
         except Exception:
             pass
+
+
+def release_server_buffers() -> None:
+    """Free the buffers that all servers keep for their next runs."""
+    load().lufqhe_server_release(None)
 
 
 def file_chunk(count: int, n: int, rank: int = 0, nodes: int = 1) -> tuple[int, int]:

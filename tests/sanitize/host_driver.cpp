@@ -1,8 +1,10 @@
 // Exercises the library's host-only code -- the CPU Crout (lucore_cpu.cpp),
-// RunInfo (run_info.cpp) and the shape-table reader (lufqhe_table.cpp) --
+// RunInfo (run_info.cpp), the shape-table reader (lufqhe_table.cpp) and the
+// pool of kept server buffers (kept_pool.hpp) --
 // under AddressSanitizer and UndefinedBehaviorSanitizer, without a GPU.  The
 // few library functions those files call are stubbed here.  Exit status 0
 // when every call returns; the sanitizers abort on the first finding.
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -10,8 +12,12 @@
 #include <string>
 #include <vector>
 
+#include <memory>
+#include <thread>
+
 #include "../../include/lucore_cpu.hpp"
 #include "../../include/lufqhe.h"
+#include "../../lion-codes_amd/csrc/kept_pool.hpp"
 
 extern "C" {
 // stubs of the kernel tables: 4 candidate shapes per n
@@ -36,6 +42,60 @@ static std::string write_tmp(const char* name, const std::string& text) {
   std::fwrite(text.data(), 1, text.size(), f);
   std::fclose(f);
   return p;
+}
+
+// The pool of buffers that idle servers keep: limits, order, and threads.
+struct FakeBuf {
+  static std::atomic<int> live;
+  int owner;
+  explicit FakeBuf(int o) : owner(o) { ++live; }
+  ~FakeBuf() { --live; }
+};
+std::atomic<int> FakeBuf::live{0};
+
+static int check_kept_pool() {
+  using Pool = lufqhe::KeptPool<FakeBuf>;
+  int o[40];
+  auto make = [](int i) { return std::make_unique<FakeBuf>(i); };
+  {
+    Pool p(100);
+    p.put(&o[0], make(0), 60);
+    p.put(&o[1], make(1), 40);
+    if (p.bytes(nullptr) != 100 || p.bytes(&o[0]) != 60 || FakeBuf::live != 2) return 20;
+    p.put(&o[2], make(2), 30);  // the oldest makes room
+    if (p.bytes(&o[0]) != 0 || p.bytes(&o[1]) != 40 || p.bytes(nullptr) != 70) return 21;
+    p.put(&o[1], make(11), 50);  // one set per owner, now the newest
+    if (p.bytes(&o[1]) != 50 || FakeBuf::live != 2) return 22;
+    p.put(&o[3], make(3), 101);  // more than the limit is not kept, and costs nobody
+    if (p.bytes(&o[3]) != 0 || p.bytes(nullptr) != 80 || FakeBuf::live != 2) return 23;
+    p.put(&o[1], make(12), 101);  // nor is the owner's old set then
+    if (p.bytes(&o[1]) != 0 || p.bytes(nullptr) != 30) return 24;
+    auto b = p.take(&o[2]);
+    if (!b || b->owner != 2 || p.take(&o[2]) || p.bytes(nullptr) != 0) return 25;
+    p.put(&o[2], std::move(b), 100);
+    if (!p.release(&o[2]) || p.release(&o[2]) || p.release(nullptr) || FakeBuf::live != 0) return 26;
+    for (int i = 0; i < 40; ++i) p.put(&o[i], make(i), 1);
+    if (p.bytes(nullptr) != Pool::kSets || FakeBuf::live != Pool::kSets || p.bytes(&o[23]) != 0 ||
+        p.bytes(&o[24]) != 1)
+      return 27;
+    if (!p.release(nullptr) || FakeBuf::live != 0 || p.bytes(nullptr) != 0) return 28;
+    std::vector<std::thread> th;
+    std::atomic<int> wrong{0};
+    for (int t = 0; t < 6; ++t)
+      th.emplace_back([&, t] {
+        for (int i = 0; i < 2000; ++i) {
+          const int k = (7 * i + t) % 20;
+          auto b = p.take(&o[k]);
+          if (b && b->owner != k) ++wrong;
+          p.put(&o[k], b ? std::move(b) : make(k), 1 + i % 30);
+          if (i % 50 == t) p.release(i % 100 == t ? nullptr : &o[k]);
+          if (p.bytes(nullptr) > 100) ++wrong;
+        }
+      });
+    for (auto& t : th) t.join();
+    if (wrong) return 29;
+  }
+  return FakeBuf::live == 0 ? 0 : 30;
 }
 
 int main(int argc, char** argv) {
@@ -69,6 +129,7 @@ int main(int argc, char** argv) {
     } catch (const LUCoreCPU::Error&) {
     }
   }
+  if (const int bad_pool = check_kept_pool()) return bad_pool;
   // invalid arguments are refused without touching memory
   if (lufqhe_cpu_crout_det(nullptr, 3, 0, 1, 1, nullptr, nullptr, nullptr, nullptr, nullptr, 1) ==
       LUFQHE_SUCCESS)

@@ -104,6 +104,77 @@ def test_sums_match_recomputed_terms(lc, dev):
     srv.close()
 
 
+RUN_A = dict(requests=120, rate=0.0, k_min=1, k_max=200, seed=9, max_batch_requests=32,
+             max_inflight=4, max_batch_dets=1 << 20)
+RUN_B = dict(RUN_A, max_batch_requests=8, max_inflight=2, max_batch_dets=4000)
+
+
+def test_kept_buffers_change_no_record(lc, dev):
+    """Runs that take the buffers of the run before them (A A), that find
+    others (B, A) and that overlap with other servers' equal a fresh server's."""
+    import threading
+    want = {}
+    for name, cfg in (("A", RUN_A), ("B", RUN_B)):
+        srv = make_server(lc)
+        want[name] = srv.run(**cfg)[1]
+        srv.close()
+
+    def work(order, failed):
+        try:
+            srv = make_server(lc)
+            for name in order:
+                srv.reset()
+                assert_same(srv.run(**(RUN_A if name == "A" else RUN_B))[1], want[name])
+                assert 0 <= lc.load().lufqhe_server_kept_bytes(None) <= 256 << 20
+                if name == "B":
+                    lc.release_server_buffers()
+            srv.close()
+        except BaseException as e:  # noqa: BLE001 -- reported by the test's own thread
+            failed.append(e)
+    failed = []
+    work("AABABB", failed)
+    assert not failed, failed
+    threads = [threading.Thread(target=work, args=(o, failed)) for o in ("ABAAB", "BAABA", "AAABB")]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    assert lc.load().lufqhe_server_kept_bytes(None) == 0
+
+
+def test_kept_buffers_are_bounded_and_given_back(lc, dev):
+    lc.release_server_buffers()
+    servers = [make_server(lc, walkers=6, perms=10) for _ in range(3)]
+    cfg = dict(requests=6, k_max=50, hbm_budget=8 << 30)
+    servers[0].run(**cfg)       # the device's first streams and pools
+    servers[0].release()
+    free0 = torch.cuda.mem_get_info()[0]
+
+    def held():
+        return free0 - torch.cuda.mem_get_info()[0]
+    for s in servers:           # 177 MiB each: the next server's set takes the room
+        s.run(**cfg)
+        kept = s.kept_bytes()
+        assert 176 << 20 < kept <= 256 << 20
+        assert lc.load().lufqhe_server_kept_bytes(None) == kept
+        assert abs(held() - kept) < 16 << 20
+    assert [s.kept_bytes() > 0 for s in servers] == [False, False, True]
+    with pytest.raises(lc.LufqheError):     # a refused run changes nothing
+        servers[2].run(requests=6, k_max=50, hbm_budget=1 << 16)
+    assert servers[2].kept_bytes() == kept
+    servers[2].release()
+    assert servers[2].kept_bytes() == 0 and held() < 16 << 20
+    # a run beyond the limit frees its buffers before it returns
+    servers[0].run(**dict(cfg, max_batch_dets=1 << 21))
+    assert lc.load().lufqhe_server_kept_bytes(None) == 0 and held() < 16 << 20
+    servers[1].run(**dict(cfg, max_batch_dets=1 << 16))
+    servers[1].close()          # and so does a server's end
+    assert lc.load().lufqhe_server_kept_bytes(None) == 0 and held() < 16 << 20
+    for s in servers:
+        s.close()
+
+
 def test_server_validation(lc, dev):
     srv = make_server(lc, walkers=6, perms=10)
     with pytest.raises(lc.LufqheError) as e:
