@@ -256,10 +256,11 @@ int32_t lufqhe_fqhe_build(const void *d_z, int64_t count, int32_t n,
  * d_A + offs[m]; LUFQHE_SOURCE_FQHE reads n[m] particle positions there and
  * builds the FQHE matrix on the device (as lufqhe_fqhe_det).  Modes:
  *   LUFQHE_MIXED_GRAPH    one launch per size with enough matrices to fill
- *                         the device (with the launch shape selected for that
- *                         size at capture time) and one per class (n <= 8,
- *                         9..16, 17..32, 33..56, 57..64) of the other sizes
- *                         (with fixed shapes), forked over the plan streams,
+ *                         the device, or alone in its class (with the launch
+ *                         shape selected for that size at capture time), and
+ *                         one per class (n <= 8, 9..16, 17..32, 33..56,
+ *                         57..64) of the other sizes (with fixed shapes, one
+ *                         per size), forked over the plan streams,
  *                         captured into one hipGraph on the first call for a
  *                         given set of pointers and source (instantiation
  *                         allocates) and replayed after; `stream` must not
@@ -292,6 +293,13 @@ int32_t lufqhe_mixed_plan_destroy(lufqhe_mixed_plan *plan);
 int32_t lufqhe_mixed_plan_buckets(const lufqhe_mixed_plan *plan, int32_t *n,
                                   int64_t *count, int32_t *stream,
                                   int32_t capacity);
+/* Kernel launches of a mode.  Fills, up to `capacity` and in the order of
+ * lufqhe_mixed_plan_buckets, each bucket's launch and whether that is its
+ * size's own kernel (1) or one it shares with its class (0); NULL arrays are
+ * skipped.  -1 for a NULL plan or an unknown mode. */
+int32_t lufqhe_mixed_plan_launches(const lufqhe_mixed_plan *plan, int32_t mode,
+                                   int32_t *launch, int32_t *own,
+                                   int32_t capacity);
 int32_t lufqhe_mixed_execute(lufqhe_mixed_plan *plan, const void *d_A,
                              void *d_mant, int32_t *d_exp, double *d_logabs,
                              double *d_phase, int32_t *d_info, int32_t source,
@@ -367,7 +375,8 @@ int32_t lufqhe_mc_lu_run(const void *h_matrices, int64_t nelem, int32_t n,
  * allows (resident state + batch buffers + 44 B per term in flight) and
  * packed into batches of at most max_batch_requests / max_batch_dets;
  * up to max_inflight batches run at once on their own streams, new ones
- * launched as earlier ones are still running.  Random numbers depend only on
+ * launched as earlier ones are still running; a batch's determinants take the
+ * launches of LUFQHE_MIXED_GRAPH, one after another.  Random numbers depend only on
  * (seed, request), so records are bit-identical for any rate or batching.
  * Results per request go to `records` (may be NULL); the walkers keep their
  * final configurations (lufqhe_server_reset restores the initial ones).

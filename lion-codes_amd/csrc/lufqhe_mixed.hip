@@ -7,8 +7,8 @@
 //     device (one allocation, made when the plan is created), so nothing is
 //     repacked;
 //   * a size with enough matrices to fill the device is one launch of its own
-//     kernel; the other sizes of a class share one launch of the class's
-//     kernel (lup_class.hpp);
+//     kernel, and so is one that has its class to itself; the other sizes of a
+//     class share one launch of the class's kernel (lup_class.hpp);
 //   * the launches are spread over the plan's streams largest-cost-first
 //     (longest-processing-time assignment on F(n) * count) and forked from /
 //     joined to the caller's stream with events, so the small ones run beside
@@ -60,9 +60,17 @@ struct lufqhe_mixed_plan {
   // one launch: a bucket by its size's own kernel, or a class of small buckets
   struct Launch {
     int bucket = -1;  // else `group`
+    int last = -1;    // the bucket `group` got last
     ClassBatch group;
     double cost = 0.0;
     int stream = 0;
+
+    bool holds(const lufqhe_mixed_plan& p, const Bucket& b) const {
+      if (bucket >= 0) return &p.buckets[bucket] == &b;
+      for (int j = 0; j < group.ca.nbuckets; ++j)
+        if (group.ca.n[j] == b.n) return true;
+      return false;
+    }
   };
   std::vector<Launch> launches;  // in launch order
   bool too_large = false;        // a bucket of 2^31 or more workgroups
@@ -145,8 +153,9 @@ bool same_out(const DetOut& a, const DetOut& b) {
 }
 
 // The plan's launches.  A bucket that fills the device's wave slots runs its
-// size's own kernel; the others of a class share one launch, largest n first.
-// Longest-processing-time assignment to the plan's streams.
+// size's own kernel; the others of a class share one launch, largest n first,
+// unless there is only one.  Longest-processing-time assignment to the plan's
+// streams.
 hipError_t build_launches(lufqhe_mixed_plan& p) {
   int cus = 0;
   const hipError_t err =
@@ -176,7 +185,10 @@ hipError_t build_launches(lufqhe_mixed_plan& p) {
     }
     if (!p.launches[o].group.add(b.n, b.start, b.count)) return hipErrorInvalidValue;
     p.launches[o].cost += b.cost;
+    p.launches[o].last = i;
   }
+  for (auto& l : p.launches)
+    if (l.bucket < 0 && l.group.alone()) l.bucket = l.last;
   std::stable_sort(p.launches.begin(), p.launches.end(),
                    [](const auto& a, const auto& b) { return a.cost > b.cost; });
   std::vector<double> load(p.nstreams, 0.0);
@@ -184,10 +196,8 @@ hipError_t build_launches(lufqhe_mixed_plan& p) {
     l.stream = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     load[l.stream] += l.cost;
     p.used[l.stream] = true;
-    if (l.bucket >= 0) p.buckets[l.bucket].stream = l.stream;
-    for (int j = 0; j < l.group.ca.nbuckets; ++j)
-      for (auto& b : p.buckets)
-        if (b.n == l.group.ca.n[j]) b.stream = l.stream;
+    for (auto& b : p.buckets)
+      if (l.holds(p, b)) b.stream = l.stream;
   }
   return hipSuccess;
 }
@@ -281,6 +291,31 @@ int32_t lufqhe_mixed_plan_buckets(const lufqhe_mixed_plan* plan, int32_t* n_out,
     if (stream_out) stream_out[i] = plan->buckets[i].stream;
   }
   return nb;
+}
+
+int32_t lufqhe_mixed_plan_launches(const lufqhe_mixed_plan* plan, int32_t mode, int32_t* launch,
+                                   int32_t* own, int32_t capacity) {
+  if (!plan || mode < LUFQHE_MIXED_GRAPH || mode > LUFQHE_MIXED_PERSISTENT) return -1;
+  const int nb = (int)plan->buckets.size();
+  if (mode == LUFQHE_MIXED_PLAIN) {  // every size's own kernel, largest n first
+    for (int i = 0; i < nb && i < capacity; ++i) {
+      if (launch)
+        launch[i] = (int32_t)std::count_if(
+            plan->buckets.begin(), plan->buckets.end(),
+            [&](const auto& b) { return b.n > plan->buckets[i].n; });
+      if (own) own[i] = 1;
+    }
+    return nb;
+  }
+  for (int i = 0; i < nb && i < capacity; ++i)
+    for (size_t j = 0; j < plan->launches.size(); ++j) {
+      const auto& l = plan->launches[j];
+      if (!l.holds(*plan, plan->buckets[i])) continue;
+      if (launch) launch[i] = (int32_t)j;
+      if (own) own[i] = l.bucket >= 0;
+      break;
+    }
+  return (int32_t)plan->launches.size();
 }
 
 int32_t lufqhe_mixed_execute(lufqhe_mixed_plan* plan, const void* d_A, void* d_mant,

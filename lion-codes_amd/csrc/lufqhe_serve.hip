@@ -16,8 +16,9 @@
 //    are still running (continuous batching);
 //  * each batch is: one prepare kernel (moves particles into per-request
 //    configuration slots, commits accepted configurations, expands per-term
-//    index tables), determinant launches (one per size that fills the device, one per
-//    class of the others) with the FQHE matrix built in the load phase, one per-request sum kernel, one small
+//    index tables), determinant launches (one per size that fills the device
+//    or has its class to itself, one per class of the others) with the FQHE
+//    matrix built in the load phase, one per-request sum kernel, one small
 //    device-to-host copy of the sums;
 //  * on completion the host applies the Metropolis rule
 //    |psi'|^2 >= u |psi|^2 (u from the request's own random stream).
@@ -394,23 +395,32 @@ struct Run {
     for (int c = kClasses - 1; c >= 0 && err == hipSuccess; --c) {
       ClassBatch cb;
       cb.cls = c;
+      auto own = [&](int n, const KernelEntry& e, int64_t blocks) {
+        BatchArgs one = a;
+        one.count = per_n[n];
+        one.ld = n;
+        one.offs += start[n];
+        one.out_idx += start[n];
+        one.perm_offs += start[n];
+        return e.launch(one, blocks, b.stream);
+      };
       for (int n = kClassHi[c]; n >= kClassLo[c] && err == hipSuccess; --n) {
         if (!per_n[n]) continue;
         const KernelEntry& e = entry_for(s->variant, n);
         const int64_t blocks = plain_blocks(e, per_n[n]);
         if (fills_device(blocks, s->cus)) {
-          BatchArgs one = a;
-          one.count = per_n[n];
-          one.ld = n;
-          one.offs += start[n];
-          one.out_idx += start[n];
-          one.perm_offs += start[n];
-          err = e.launch(one, blocks, b.stream);
+          err = own(n, e, blocks);
         } else if (!cb.add(n, start[n], per_n[n])) {
           err = hipErrorInvalidValue;
         }
       }
-      if (cb.tasks && err == hipSuccess) err = cb.launch(s->variant, a, b.stream);
+      if (err == hipSuccess && cb.alone()) {
+        const int n = cb.ca.n[0];
+        const KernelEntry& e = entry_for(s->variant, n);
+        err = own(n, e, plain_blocks(e, per_n[n]));
+      } else if (err == hipSuccess && cb.tasks) {
+        err = cb.launch(s->variant, a, b.stream);
+      }
     }
     if (err == hipSuccess) {
       hipLaunchKernelGGL(serve_sum_kernel, dim3(nr), dim3(64), 0, b.stream, b.d_desc, b.d_mant,

@@ -82,7 +82,7 @@ extern SmallLaunch g_small[kClassVariants][kMaxN + 1];
 
 // Whether a launch of `blocks` one-wave workgroups fills the device's wave
 // slots at two waves per SIMD.  From there on a size's own kernel wins, below
-// it a launch shared with the other sizes of the class: with all of a batch
+// it a launch shared with other sizes of the class: with all of a batch
 // of one size the class kernels take 1-5% longer (n <= 32) to 10-20% longer
 // (n >= 33, where they spill more), but 32768 matrices of n = 10..40 in 31
 // launches on four streams took 298 us and in shared ones 238.
@@ -93,9 +93,13 @@ constexpr bool fills_device(int64_t blocks, int cus) { return blocks >= (int64_t
 struct ClassBatch {
   int cls = 0;
   int64_t tasks = 0;
-  double cost = 0.0;
-  int stream = 0;
   ClassArgs ca{};
+
+  // A size that shares with no other runs its own kernel: the class kernel
+  // takes longer for it (graph replay of one size, us, class | own: 1000 x
+  // n = 24 26.0 | 25.1, 1900 x n = 57 101 | 93, 1900 x n = 64 115 | 109) and
+  // there is no launch to save.
+  bool alone() const { return ca.nbuckets == 1; }
 
   // matrices first .. first+count-1 of the index tables have side n
   bool add(int n, int64_t first, int64_t count) {

@@ -102,6 +102,8 @@ def load() -> ctypes.CDLL:
     lib.lufqhe_mixed_plan_destroy.argtypes = [_vp]
     lib.lufqhe_mixed_plan_buckets.restype = _i32
     lib.lufqhe_mixed_plan_buckets.argtypes = [_vp, _vp, _vp, _vp, _i32]
+    lib.lufqhe_mixed_plan_launches.restype = _i32
+    lib.lufqhe_mixed_plan_launches.argtypes = [_vp, _i32, _vp, _vp, _i32]
     lib.lufqhe_mixed_execute.restype = _i32
     lib.lufqhe_mixed_execute.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _vp]
     lib.lufqhe_fqhe_det.restype = _i32
@@ -660,6 +662,16 @@ class MixedPlan:
         s = np.empty(nb, np.int32)
         _lib.lufqhe_mixed_plan_buckets(self._h, n.ctypes.data, c.ctypes.data, s.ctypes.data, nb)
         return list(zip(n.tolist(), c.tolist(), s.tolist()))
+
+    def launches(self, mode: str = "graph"):
+        """(kernel launches of the mode, {n: (launch, whether it is the size's
+        own kernel)})."""
+        import numpy as np
+        ns = [b[0] for b in self.buckets()]
+        at, own = np.empty(len(ns), np.int32), np.empty(len(ns), np.int32)
+        count = _lib.lufqhe_mixed_plan_launches(self._h, MIXED_MODES[mode], at.ctypes.data,
+                                                own.ctypes.data, len(ns))
+        return count, {n: (int(a), bool(o)) for n, a, o in zip(ns, at, own)}
 
     def execute(self, flat: torch.Tensor, out: DetResult, mode: str = "graph",
                 stream: torch.cuda.Stream | None = None, source: str = "matrix") -> DetResult:
