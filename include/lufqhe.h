@@ -269,9 +269,11 @@ int32_t lufqhe_fqhe_build(const void *d_z, int64_t count, int32_t n,
  *   LUFQHE_MIXED_STREAMS  the same forked launches, issued directly;
  *   LUFQHE_MIXED_PLAIN    one launch per size with the shape selected for it,
  *                         one after another on `stream`;
- *   LUFQHE_MIXED_PERSISTENT  the same as GRAPH; a plan with 2^31 or more
- *                         workgroups of one size refuses it
- *                         (LUFQHE_ERROR_UNSUPPORTED).
+ *   LUFQHE_MIXED_PERSISTENT  one launch per class, large sizes included: at
+ *                         most five whatever the batch (more only beyond 2^26
+ *                         workgroups of a class), captured and replayed like
+ *                         GRAPH.  A plan with 2^31 or more workgroups of a
+ *                         class refuses it (LUFQHE_ERROR_UNSUPPORTED).
  * A plan is not re-entrant: one execute at a time per plan, on the device
  * that was current when it was created (else LUFQHE_ERROR_INVALID_VALUE). */
 #define LUFQHE_MIXED_GRAPH 0

@@ -14,11 +14,12 @@
 //     joined to the caller's stream with events, so the small ones run beside
 //     the large ones instead of after them;
 //   * the whole fork/launch/join sequence is captured once into a hipGraph
-//     and replayed: one graph launch per batch.  PERSISTENT is the same
-//     sequence.
+//     and replayed: one graph launch per batch.
 // A launch per size leaves wave slots empty when its bucket is small, and each
 // waited for the one before it on its stream: 32768 FQHE matrices of 31 sizes
 // took 298 us that way and take 239, 2675 matrices of 24 sizes 353 and 130.
+// Mode PERSISTENT is captured like GRAPH and has class launches only, five at
+// most whatever the batch.
 // Mode PLAIN runs each size's own kernel one after another on the caller's
 // stream: the uniform-launch-per-size form the others are compared with.
 #include <hip/hip_runtime.h>
@@ -56,7 +57,6 @@ struct lufqhe_mixed_plan {
   hipStream_t streams[LUFQHE_MIXED_MAX_STREAMS] = {};
   hipEvent_t fork = nullptr;
   hipEvent_t join[LUFQHE_MIXED_MAX_STREAMS] = {};
-  bool used[LUFQHE_MIXED_MAX_STREAMS] = {};  // streams a launch is assigned to
   // one launch: a bucket by its size's own kernel, or a class of small buckets
   struct Launch {
     int bucket = -1;  // else `group`
@@ -73,12 +73,14 @@ struct lufqhe_mixed_plan {
     }
   };
   std::vector<Launch> launches;  // in launch order
-  bool too_large = false;        // a bucket of 2^31 or more workgroups
+  std::vector<Launch> shared;    // PERSISTENT: class launches only
+  bool too_large = false;        // a class of 2^31 or more tasks
   // captured graph and what it was captured for
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   const void* g_A = nullptr;
   int g_src = 0;
+  int g_mode = -1;
   DetOut g_out{};
 
   ~lufqhe_mixed_plan() {
@@ -126,21 +128,24 @@ BatchArgs class_args(const lufqhe_mixed_plan& p, const void* d_A, int src, const
 }
 
 // Fork from `stream`, the launches on the plan's streams, join back.
-hipError_t issue_forked(const lufqhe_mixed_plan& p, const void* d_A, int src,
-                        const DetOut& out, hipStream_t stream) {
+hipError_t issue_forked(const lufqhe_mixed_plan& p,
+                        const std::vector<lufqhe_mixed_plan::Launch>& launches, const void* d_A,
+                        int src, const DetOut& out, hipStream_t stream) {
   const BatchArgs args = class_args(p, d_A, src, out);
   auto launch = [&](const lufqhe_mixed_plan::Launch& l, hipStream_t s) {
     return l.bucket >= 0 ? launch_bucket(p, p.buckets[l.bucket], d_A, src, out, s)
                          : l.group.launch(p.variant, args, s);
   };
-  if (p.launches.size() == 1) return launch(p.launches[0], stream);
+  if (launches.size() == 1) return launch(launches[0], stream);
+  bool used[LUFQHE_MIXED_MAX_STREAMS] = {};
+  for (const auto& l : launches) used[l.stream] = true;
   hipError_t err = hipEventRecord(p.fork, stream);
   for (int s = 0; s < p.nstreams && err == hipSuccess; ++s)
-    if (p.used[s]) err = hipStreamWaitEvent(p.streams[s], p.fork, 0);
-  for (const auto& l : p.launches)
+    if (used[s]) err = hipStreamWaitEvent(p.streams[s], p.fork, 0);
+  for (const auto& l : launches)
     if (err == hipSuccess) err = launch(l, p.streams[l.stream]);
   for (int s = 0; s < p.nstreams && err == hipSuccess; ++s) {
-    if (!p.used[s]) continue;
+    if (!used[s]) continue;
     err = hipEventRecord(p.join[s], p.streams[s]);
     if (err == hipSuccess) err = hipStreamWaitEvent(stream, p.join[s], 0);
   }
@@ -152,15 +157,12 @@ bool same_out(const DetOut& a, const DetOut& b) {
          a.info == b.info && a.piv == b.piv;
 }
 
-// The plan's launches.  A bucket that fills the device's wave slots runs its
-// size's own kernel; the others of a class share one launch, largest n first,
-// unless there is only one.  Longest-processing-time assignment to the plan's
-// streams.
-hipError_t build_launches(lufqhe_mixed_plan& p) {
-  int cus = 0;
-  const hipError_t err =
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p.device);
-  if (err != hipSuccess) return err;
+// The plan's launches.  With `own`, a bucket that fills the device's wave slots
+// runs its size's own kernel; the others of a class share one launch, largest n
+// first, unless there is only one.  Without, every bucket shares its class's.
+// Longest-processing-time assignment to the plan's streams.
+std::vector<lufqhe_mixed_plan::Launch> plan_launches(const lufqhe_mixed_plan& p, int cus, bool own) {
+  std::vector<lufqhe_mixed_plan::Launch> out;
   std::vector<int> order(p.buckets.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
   std::sort(order.begin(), order.end(),
@@ -169,36 +171,55 @@ hipError_t build_launches(lufqhe_mixed_plan& p) {
   std::fill(open, open + kClasses, -1);
   for (int i : order) {
     const auto& b = p.buckets[i];
-    const int64_t blocks = plain_blocks(entry_for(p.variant, b.n), b.count);
-    p.too_large = p.too_large || blocks > INT32_MAX;
-    if (fills_device(blocks, cus)) {
-      p.launches.emplace_back();
-      p.launches.back().bucket = i;
-      p.launches.back().cost = b.cost;
+    if (own && fills_device(plain_blocks(entry_for(p.variant, b.n), b.count), cus)) {
+      out.emplace_back();
+      out.back().bucket = i;
+      out.back().cost = b.cost;
       continue;
     }
     int& o = open[size_class(b.n)];
-    if (o < 0) {
-      o = (int)p.launches.size();
-      p.launches.emplace_back();
-      p.launches.back().group.cls = size_class(b.n);
+    for (int64_t done = 0; done < b.count;) {
+      int64_t took = 0;
+      if (o >= 0) took = out[o].group.add(b.n, b.start + done, b.count - done);
+      if (took == 0) {  // the class's first bucket, or a grid is full
+        o = (int)out.size();
+        out.emplace_back();
+        out[o].group.cls = size_class(b.n);
+        continue;
+      }
+      out[o].cost += b.cost * ((double)took / b.count);
+      out[o].last = i;
+      done += took;
     }
-    if (!p.launches[o].group.add(b.n, b.start, b.count)) return hipErrorInvalidValue;
-    p.launches[o].cost += b.cost;
-    p.launches[o].last = i;
   }
-  for (auto& l : p.launches)
-    if (l.bucket < 0 && l.group.alone()) l.bucket = l.last;
-  std::stable_sort(p.launches.begin(), p.launches.end(),
+  if (own)
+    for (auto& l : out)
+      if (l.bucket < 0 && l.group.alone()) l.bucket = l.last;
+  std::stable_sort(out.begin(), out.end(),
                    [](const auto& a, const auto& b) { return a.cost > b.cost; });
   std::vector<double> load(p.nstreams, 0.0);
-  for (auto& l : p.launches) {
+  for (auto& l : out) {
     l.stream = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     load[l.stream] += l.cost;
-    p.used[l.stream] = true;
+  }
+  return out;
+}
+
+hipError_t build_launches(lufqhe_mixed_plan& p) {
+  int cus = 0;
+  const hipError_t err =
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p.device);
+  if (err != hipSuccess) return err;
+  p.launches = plan_launches(p, cus, true);
+  p.shared = plan_launches(p, cus, false);
+  int64_t tasks[kClasses] = {};
+  for (const auto& l : p.shared) {
+    tasks[l.group.cls] += l.group.tasks;
+    p.too_large = p.too_large || tasks[l.group.cls] > INT32_MAX;
+  }
+  for (const auto& l : p.launches)
     for (auto& b : p.buckets)
       if (l.holds(p, b)) b.stream = l.stream;
-  }
   return hipSuccess;
 }
 
@@ -307,15 +328,16 @@ int32_t lufqhe_mixed_plan_launches(const lufqhe_mixed_plan* plan, int32_t mode, 
     }
     return nb;
   }
+  const auto& launches = mode == LUFQHE_MIXED_PERSISTENT ? plan->shared : plan->launches;
   for (int i = 0; i < nb && i < capacity; ++i)
-    for (size_t j = 0; j < plan->launches.size(); ++j) {
-      const auto& l = plan->launches[j];
+    for (size_t j = 0; j < launches.size(); ++j) {
+      const auto& l = launches[j];
       if (!l.holds(*plan, plan->buckets[i])) continue;
       if (launch) launch[i] = (int32_t)j;
       if (own) own[i] = l.bucket >= 0;
       break;
     }
-  return (int32_t)plan->launches.size();
+  return (int32_t)launches.size();
 }
 
 int32_t lufqhe_mixed_execute(lufqhe_mixed_plan* plan, const void* d_A, void* d_mant,
@@ -343,11 +365,11 @@ int32_t lufqhe_mixed_execute(lufqhe_mixed_plan* plan, const void* d_A, void* d_m
       if (err != hipSuccess) break;
     }
   } else if (mode == LUFQHE_MIXED_STREAMS) {
-    err = issue_forked(*plan, d_A, src, out, stream);
+    err = issue_forked(*plan, plan->launches, d_A, src, out, stream);
   } else if (mode == LUFQHE_MIXED_GRAPH || mode == LUFQHE_MIXED_PERSISTENT) {
     if (stream == nullptr) return LUFQHE_ERROR_INVALID_VALUE;  // no capture on stream 0
     if (mode == LUFQHE_MIXED_PERSISTENT && plan->too_large) return LUFQHE_ERROR_UNSUPPORTED;
-    if (!plan->exec || plan->g_A != d_A || plan->g_src != src ||
+    if (!plan->exec || plan->g_mode != mode || plan->g_A != d_A || plan->g_src != src ||
         !same_out(plan->g_out, out)) {
       if (plan->exec) (void)hipGraphExecDestroy(plan->exec);
       if (plan->graph) (void)hipGraphDestroy(plan->graph);
@@ -355,7 +377,9 @@ int32_t lufqhe_mixed_execute(lufqhe_mixed_plan* plan, const void* d_A, void* d_m
       plan->graph = nullptr;
       if (err == hipSuccess) err = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
       if (err == hipSuccess) {
-        const hipError_t e2 = issue_forked(*plan, d_A, src, out, stream);
+        const hipError_t e2 =
+            issue_forked(*plan, mode == LUFQHE_MIXED_PERSISTENT ? plan->shared : plan->launches,
+                         d_A, src, out, stream);
         err = hipStreamEndCapture(stream, &plan->graph);
         if (e2 != hipSuccess) err = e2;
       }
@@ -363,6 +387,7 @@ int32_t lufqhe_mixed_execute(lufqhe_mixed_plan* plan, const void* d_A, void* d_m
       if (err == hipSuccess) {
         plan->g_A = d_A;
         plan->g_src = src;
+        plan->g_mode = mode;
         plan->g_out = out;
       }
     }

@@ -410,7 +410,7 @@ struct Run {
         const int64_t blocks = plain_blocks(e, per_n[n]);
         if (fills_device(blocks, s->cus)) {
           err = own(n, e, blocks);
-        } else if (!cb.add(n, start[n], per_n[n])) {
+        } else if (cb.add(n, start[n], per_n[n]) != per_n[n]) {
           err = hipErrorInvalidValue;
         }
       }

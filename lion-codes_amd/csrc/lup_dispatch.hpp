@@ -82,15 +82,16 @@ extern SmallLaunch g_small[kClassVariants][kMaxN + 1];
 
 // Whether a launch of `blocks` one-wave workgroups fills the device's wave
 // slots at two waves per SIMD.  From there on a size's own kernel wins, below
-// it a launch shared with other sizes of the class: with all of a batch
-// of one size the class kernels take 1-5% longer (n <= 32) to 10-20% longer
-// (n >= 33, where they spill more), but 32768 matrices of n = 10..40 in 31
-// launches on four streams took 298 us and in shared ones 238.
+// it a launch shared with other sizes of the class: with all of a batch of one
+// size the class kernels take 2-5% longer (n <= 32), 5-7% (n = 36..48), 6-15%
+// (n = 57..64) and only at n = 52 and 56 no longer, but 32768 matrices of n =
+// 10..40 in 31 launches on four streams took 298 us and in shared ones 238.
 constexpr bool fills_device(int64_t blocks, int cus) { return blocks >= (int64_t)cus * 8; }
 
 // One class launch being put together: the buckets of its class, added
 // largest n first.
 struct ClassBatch {
+  static constexpr int64_t kMostTasks = (int64_t{1} << 26) - 1;  // 64 threads each: a grid holds 2^32
   int cls = 0;
   int64_t tasks = 0;
   ClassArgs ca{};
@@ -101,15 +102,20 @@ struct ClassBatch {
   // there is no launch to save.
   bool alone() const { return ca.nbuckets == 1; }
 
-  // matrices first .. first+count-1 of the index tables have side n
-  bool add(int n, int64_t first, int64_t count) {
+  // Matrices first .. first+count-1 of the index tables have side n: how many
+  // of them the launch takes (whole tasks, up to its grid's limit).
+  int64_t add(int n, int64_t first, int64_t count) {
+    const int g = class_group(n);
+    const int64_t room = (kMostTasks - tasks) * g;
+    if (count > room) count = room;
+    if (count <= 0) return 0;
     const int b = ca.nbuckets++;
     ca.n[b] = n;
     ca.task[b] = (int32_t)tasks;
     ca.first[b] = first;
     ca.count[b] = count;
-    tasks += (count + class_group(n) - 1) / class_group(n);
-    return tasks <= INT32_MAX;  // a grid's size
+    tasks += (count + g - 1) / g;
+    return count;
   }
   hipError_t launch(int variant, const BatchArgs& args, hipStream_t s) const {
     ClassArgs a = ca;

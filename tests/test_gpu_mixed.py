@@ -1,7 +1,7 @@
 """GPU parity of mixed-size batches (one flat buffer, n = 1..64 per matrix).
 
-Every mode -- one hipGraph replayed, forked streams, plain per-size launches,
-persistent class kernels draining device work queues -- must give the
+Every mode -- one hipGraph replayed (own and class kernels), forked streams,
+plain per-size launches, class kernels for every size -- must give the
 oracle's determinants bit for bit at each matrix's own index. The graphs are
 replayed several times with eager work and synchronisation in between; every
 replay is checked.
@@ -69,10 +69,9 @@ def test_graph_replays_with_eager_work_between(lc, orc, wl, dev, mode):
 
 
 def test_persistent_new_pointers_and_single_class(lc, orc, wl, dev):
-    """Changing the output buffers re-captures the persistent graph with new
-    per-bucket arguments, and switching back works; a batch whose sizes all
-    fall in one class (n = 3..9) uses one class kernel; modes alternate on
-    one plan."""
+    """Changing the output buffers or the mode captures the graph again, and
+    switching back works; a batch whose sizes fall in two classes (n = 3..9)
+    has two class launches in persistent mode, one with n = 1..64 five."""
     side = torch.cuda.Stream()
     for lo, hi, count in ((3, 9, 700), (1, 64, 1200)):
         flat, ns, offs = mixed_input(wl, count, seed=lo + hi, lo=lo, hi=hi)
@@ -80,6 +79,8 @@ def test_persistent_new_pointers_and_single_class(lc, orc, wl, dev):
         d = flat.to(dev)
         o = orc.mirror_mixed(flat_np, ns, offs, "crout_ref", "fused")
         plan = lc.MixedPlan(ns, offs, nstreams=2)
+        launches, at = plan.launches("persistent")
+        assert launches == (2 if hi == 9 else 5) and not any(own for _, own in at.values())
         r1 = lc.alloc_result(len(ns), 64, dev)
         r2 = lc.alloc_result(len(ns), 64, dev)
         for res, mode in ((r1, "persistent"), (r2, "persistent"), (r1, "graph"),
@@ -158,7 +159,9 @@ def test_own_and_class_launches_of_one_plan(lc, orc, dev, policy):
         plan.execute(flat, want, mode="plain", stream=side)
     side.synchronize()
     sample_check(orc, flat, ns, offs, want, policy)
-    for mode in ("streams", "graph"):
+    shared, class_at = plan.launches("persistent")
+    assert shared == 5 and not any(own for _, own in class_at.values())
+    for mode in ("streams", "graph", "persistent"):
         res = lc.alloc_result(len(ns), 64, dev)
         res.mant.zero_()
         with torch.cuda.stream(side):
@@ -227,13 +230,15 @@ def test_config4_full_size(lc, orc, wl, dev):
     sub = np.concatenate([flat_cpu[offs[i]:offs[i] + ns[i] ** 2] for i in idx])
     o = orc.mirror_mixed(sub, sub_ns, sub_offs, "crout_ref", "fused")
     assert np.array_equal(bits(res.mant.cpu().numpy()[idx]), bits(o["mant"]))
-    # the persistent class kernels give the same bits for every matrix
-    rp = lc.alloc_result(len(ns), 64, dev)
-    with torch.cuda.stream(side):
-        plan.execute(flat, rp, mode="persistent", stream=side)
-    side.synchronize()
-    assert torch.equal(rp.mant.view(torch.float64), res.mant.view(torch.float64))
-    assert torch.equal(rp.exp, res.exp) and torch.equal(rp.info, res.info)
+    # the sizes' own kernels and the class kernels give the same bits for every matrix
+    assert all(own for _, own in plan.launches("plain")[1].values())
+    assert not any(own for _, own in plan.launches("persistent")[1].values())
+    for mode in ("plain", "persistent"):
+        rp = lc.alloc_result(len(ns), 64, dev)
+        with torch.cuda.stream(side):
+            plan.execute(flat, rp, mode=mode, stream=side)
+        side.synchronize()
+        assert_same_results(rp, res, mode)
     t = orc.truth_mixed(sub, sub_ns, sub_offs)
     la = res.logabs.cpu().numpy()[idx]
     ph = res.phase.cpu().numpy()[idx]
