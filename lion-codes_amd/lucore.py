@@ -146,6 +146,11 @@ def load() -> ctypes.CDLL:
                                      ctypes.POINTER(McStats)]
     lib.lufqhe_fqhe_build.restype = _i32
     lib.lufqhe_fqhe_build.argtypes = [_vp, _i64, _i32, _i64, _vp, _vp, _vp]
+    # Loading a library with thread-locals puts glibc's lookup of every other
+    # library's on its slow path until this thread uses the newest ones
+    # (torch.empty 1.24 against 0.98 us, det_batched of two 10x10 matrices with
+    # its results allocated 16.6 against 14.4): use the library's once.
+    lib.lufqhe_last_hip_error()
     _lib = lib
     apply_shape_table()
     return lib
