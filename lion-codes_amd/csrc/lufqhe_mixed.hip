@@ -194,7 +194,8 @@ std::vector<lufqhe_mixed_plan::Launch> plan_launches(const lufqhe_mixed_plan& p,
   }
   if (own)
     for (auto& l : out)
-      if (l.bucket < 0 && l.group.alone()) l.bucket = l.last;
+      if (l.bucket < 0 && l.group.alone() && l.group.ca.count[0] == p.buckets[l.last].count)
+        l.bucket = l.last;
   std::stable_sort(out.begin(), out.end(),
                    [](const auto& a, const auto& b) { return a.cost > b.cost; });
   std::vector<double> load(p.nstreams, 0.0);
