@@ -86,6 +86,9 @@ struct lufqhe_mixed_plan {
   ~lufqhe_mixed_plan() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
+    // HIP releases an executable graph at the next synchronisation: that comes
+    // before the end of the streams and events it was captured from.
+    if (exec) (void)hipDeviceSynchronize();
     for (int s = 0; s < nstreams; ++s) {
       if (join[s]) (void)hipEventDestroy(join[s]);
       if (streams[s]) (void)hipStreamDestroy(streams[s]);
