@@ -71,7 +71,12 @@ extern ClassLaunch g_class[kClassVariants][kClasses];
 // n = 32 15.1 / 18.3, n = 56 29.2 / 36.1, n = 64 34.9 / 42.2 at 48 matrices;
 // n = 32 17.2 / 19.5 at 1024 and 23.5 / 22.4 at 2048; n = 64 35.4 / 42.6 at 256 and
 // 48.7 / 44.1 at 512.  At n = 33..48 two waves gained at most 9% and lost at
-// 512 matrices.
+// 512 matrices.  n <= 16 has no such route.  Measured there, us a call back to
+// back, {8,1,1} / {16,1,1} / panel kernel with one / two matrices per wave: n =
+// 16 13.0 / 10.4 / 10.4 / 10.3 at 2 matrices, 13.1 / 10.4 / 10.6 / 10.4 at 1000,
+// 14.7 / 14.1 / 18.1 / 13.5 at 4096, 17.0 / 18.5 / 31.0 / 19.6 at 8192; n =
+// 8..12 10.1 to 10.9 with any of them up to 4096, which is the host's time of a
+// call (the kernels take 6.5 to 9.7, the panel ones 4.9 to 7.3 up to 1000).
 constexpr int small_waves(int n) { return n < 17 ? 0 : n <= 32 ? 1 : n <= 48 ? 0 : 2; }
 constexpr bool small_batch(int n, int64_t count, int cus) {
   return count <= (n <= 32 ? 4 : 1) * (int64_t)cus;

@@ -34,9 +34,9 @@
 // not overlap, and alternating them is slower than running them in runs), so
 // a step costs its issue: an n = 32 wave (two matrices) issues 3814
 // instructions, 312 of them MFMAs of 16 cycles, where lup_det_kernel issued
-// 6167; at two waves per SIMD they fill 72% of the cycles and LDS is busy for
-// 51%.  The rest is the latency of the serial search, pivot row and
-// reciprocal.  65536 x n = 32: 475 -> 396 us; above n = 56 the tile leaves
+// 6167; at two waves per SIMD they fill 73% of the cycles and LDS is busy for
+// 45%.  The rest is the latency of the serial search, pivot row and
+// reciprocal.  65536 x n = 32: 482 -> 398 us; above n = 56 the tile leaves
 // room for one wave per SIMD only (n = 64: 82 -> 49 ns per determinant).
 //
 // H = 2 (one matrix, two waves) is for batches with fewer matrices than CUs,
@@ -78,7 +78,7 @@ constexpr int panel_lds(int n, int g, int h) {
 // only the places that take a row read), the row's state by ds_bpermute.  All
 // later panels then update, write and read one slot less.  Measured with and
 // without, ns per determinant: n = 32 6.55 / 6.88 (with pivot rows still passed
-// through LDS; now 6.33), n = 40 13.4 / 14.6, n = 48 18.5 / 19.7, n = 52
+// through LDS; now 6.23), n = 40 13.4 / 14.6, n = 48 18.5 / 19.7, n = 52
 // 24.1 / 30.8 (one slot less after the first panel, and so no spills at two
 // waves per SIMD), n = 64 48.7 / 50.4.  kMinPanelsLeft = 1, 3 and 4 are within
 // 1% at n = 26..64.
@@ -458,7 +458,7 @@ __device__ __forceinline__ void panel_task(const BatchArgs& args, int64_t task,
           // instructions per panel, but no write that a read then waits for:
           // LDS moves 64 B per clock and CU on writes and was busy for 70% of
           // n = 32; 6.59 -> 6.33 ns per determinant there, 5.06 -> 4.90 at
-          // n = 26).  With one matrix per wave v_readlane is as fast (n = 40)
+          // n = 26; 45% now, with the areas' spacing too).  With one matrix per wave v_readlane is as fast (n = 40)
           // or faster (n = 64, 4%).
           int pl[G];
 #pragma unroll
